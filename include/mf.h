@@ -195,8 +195,10 @@ int mf_matrix_get_info(mf_matrix m, mf_matrix_info *info);
  * form where every tile row has few enough tiles (B = 8: 8, 16: 16, 32: 8),
  * else the four-byte column; with the two- and four-byte forms, a class slab
  * whose rows share their column offsets (stencils) stores one table of
- * offsets instead of an index per entry (pattern slab).  1, 2 or 4 = that
- * form where it fits, else the next wider one, and no pattern slabs.
+ * offsets instead of an index per entry (pattern slab), and where all rows
+ * of the matrix draw from one short table of offsets and the layout holds one
+ * class, the solvers run on planes of values without indices.  1, 2 or 4 = that
+ * form where it fits, else the next wider one, and no pattern slabs or planes.
  * Layouts already built are released.  Results are bit-identical across
  * forms.  No reference counterpart (the reference stores four-byte columns
  * only). */
@@ -277,8 +279,9 @@ typedef struct {
     double pad_factor;   /* stored slab entries / nonzeros of the natural FP64 layout */
     int sync_deps;       /* BiCGSTAB neighbour syncs: most workgroups one waits
                             for after a publish; -1: grid barriers */
-    int streamed;        /* 1: the Krylov vectors lived in HBM (systems beyond
-                            register/LDS residency, or opts.vectors) */
+    int streamed;        /* 1: Krylov vectors lived in HBM (systems beyond
+                            register/LDS residency, or opts.vectors; on stencil
+                            planes up to 36 rows per thread x alone) */
     int fallback;        /* 1: the solve on lossy tiles diverged, broke down or
                             hit maxit, and was redone on the FP64 layout (its
                             time and iterations are included); batched: the

@@ -50,6 +50,8 @@ struct DevL {
     const uint8_t *split = nullptr;
 };
 
+constexpr int STENCIL_MAX = 32;  // offsets of a stencil matrix's table (stencil.h)
+
 // Sum over the S-lane segment of this lane (S a power of two within the
 // lane group, every lane of the segment active); the segment's first lane
 // keeps it, the other lanes return 0.

@@ -9,6 +9,7 @@
 
 namespace mf {
 
+struct StencilTable;  // stencil.h
 int hip_fail(hipError_t e, const char *what);
 #define MF_HIP(call)                                         \
     do {                                                     \
@@ -37,6 +38,11 @@ struct Layout {
     double bytes_actual = 0.0;  // bytes the layout occupies (+ gather + y)
     long long pattern_slabs = 0;  // (tile row, class) slabs in pattern form
     const uint8_t *split = nullptr;  // the matrix's split tile rows (not owned)
+    // stencil planes beside the slabs, when the matrix and the layout qualify
+    // (ensure_planes; stencil.h)
+    uint8_t *planes = nullptr;
+    int planes_cls = -1;
+    bool planes_tried = false;
     DevL view(const int *tile_ptr) const { return DevL{tile_ptr, trh, stc, blob, split}; }
     void release();
 };
@@ -85,6 +91,10 @@ struct mf_matrix_s {
     uint8_t *d_rowtmp = nullptr;
     double *d_Blockcsr_Val = nullptr;
     float *d_Blockcsr_Val_Low = nullptr;
+    // offset table of a stencil matrix on the device, and its length (-1 not
+    // looked for yet, 0 no stencil)
+    mf::StencilTable *d_st = nullptr;
+    int st_L = -1;
     // compute layouts and scratch
     mf::Layout L64, Lmix;
     mf::Workspace ws;
@@ -109,6 +119,10 @@ int build_reference_tiles(mf_matrix m);              // tiles.hip
 // pattern: pattern slabs where they fit (automatic index form only)
 int build_layout(mf_matrix m, Layout &L, double tau, int allow_mask, int want_iw = 0,
                  bool pattern = true);  // tiles.hip
+// the stencil planes of a built layout in the automatic index form, where the
+// matrix is a stencil and the layout holds one class (L.planes stays null
+// where not)
+int ensure_planes(mf_matrix m, Layout &L);  // tiles.hip
 // fits bit 0: the one-byte slot form fits, bit 1: the two-byte form fits
 int index_fits(mf_matrix m, int *fits);  // tiles.hip
 // the width used for a request (0 automatic: two bytes, else one, else four;

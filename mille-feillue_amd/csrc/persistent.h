@@ -9,11 +9,13 @@
 #include <type_traits>
 
 #include "mf_matrix.h"
+#include "stencil.h"
 
 namespace mf {
 
 // --------------------------------------------------------- solver kernels
 constexpr int SYNC_K = 5;  // values per grid allreduce, at most
+constexpr int X_REGS_ROWS = 16;   // rows per thread up to which the resident CG keeps x in registers
 constexpr int LDS_GATHER = 2048;  // rows of a one-workgroup solve gathered from LDS
 // A true-residual pass on a lossy layout whose squared norm exceeds the best
 // earlier one by this factor (the norm grew 4x while the recurrence claimed
@@ -25,8 +27,11 @@ struct SolveArgs {
     DevL L;
     unsigned long long blob_bytes;  // bytes of L's slab blob
     DevL L64;          // FP64 layout for the true-residual passes of a lossy layout
-    int use64;         // 1: passes use L64 (headers read from L64), else L
+    int use64;         // 1: passes use L64 (headers read from L64) or pl64, else L or pl
+    Planes pl, pl64;   // stencil kernels: the layout's planes, and the FP64 ones (use64)
+    const int *off;    // and the offset table
     int tilem, G, trw;
+    int nrows, crows;  // rows of the system and of a chunk (tilem and trw tile rows)
     const double *b;
     double *x;
     double *g64;       // published Krylov vector (FP64)
@@ -52,6 +57,12 @@ struct SolveArgs {
     double *vec;
     long long vstride;
 };
+
+}  // namespace mf
+
+#include "stencil_product.h"
+
+namespace mf {
 
 // Phase clock of block 0 (diagnostic; enabled when A.phase is set).
 struct PhaseClock {
@@ -118,8 +129,13 @@ struct Reducer {
     int *s_flag;
     unsigned ep = 0;
 
-    template <int N>
-    __device__ bool allreduce(const SolveArgs &A, double (&v)[N], bool publish)
+    // meanwhile: work of this workgroup's threads done between its words and
+    // the poll
+    struct Nothing {
+        __device__ void operator()() const {}
+    };
+    template <int N, typename F = Nothing>
+    __device__ bool allreduce(const SolveArgs &A, double (&v)[N], bool publish, F meanwhile = F())
     {
         static_assert(N >= 1 && N <= K, "reducer width");
         const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -137,6 +153,7 @@ struct Reducer {
         unsigned long long *st = stamp ? A.phase + 16 + (size_t)(ep - PHASE_EP0) * 2 * A.G + 2 * blockIdx.x : nullptr;
         if (stamp) st[0] = wall_clock64();
         if (A.G == 1) {
+            meanwhile();
             // one workgroup: the reduction stays in LDS; published entries
             // are read back through this CU's L1, which the acquire refreshes
             if (tid < 64) {
@@ -153,9 +170,9 @@ struct Reducer {
             for (int k = 0; k < N; k++) v[k] = s_bc[k];
             return true;
         }
+        const unsigned G = (unsigned)A.G;
+        unsigned long long *W = A.slots + (size_t)(ep % SLOT_BUFS) * G * SLOT_WORDS;
         if (tid < 64) {
-            const unsigned G = (unsigned)A.G;
-            unsigned long long *W = A.slots + (size_t)(ep % SLOT_BUFS) * G * SLOT_WORDS;
             __builtin_amdgcn_s_waitcnt(0);  // the emptying of this line has completed
             if (lane < N) {
                 double s = 0.0;
@@ -164,6 +181,9 @@ struct Reducer {
                                    (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
             }
+        }
+        meanwhile();
+        if (tid < 64) {
             double acc[N];
             long long spins = 0;
             int ab = 0;
@@ -356,6 +376,72 @@ __device__ bool stage_chunk(const SolveArgs &A, int tr0, int tr1, int TRW, int4 
     return lds;
 }
 
+// The slab product of a resident kernel: tiles of B rows, indices of IW bytes,
+// the classes in CM.
+template <int B, int IW, int CM = CM_ALL> struct Slabs {
+    static constexpr bool r_regs = false;
+    static constexpr bool lds_tags = true;  // slabs in LDS or in HBM known at compile time
+    template <int TPB, int RPT, int VECS, int VREGS> struct Op {
+        static constexpr int GPB = TPB / B, NR = spmv_rows(RPT, IW), TRW = RPT * GPB, LSB = lds_slab_bytes(RPT);
+        struct Shared {
+            // headers of the block's tile rows, loaded once: the per-iteration
+            // SpMV then issues the tile-column word and the slab loads together
+            int4 h[2 * TRW];
+            int t0[TRW + 1];
+            // small chunks keep their slabs in LDS too
+            alignas(16) uint8_t slab[LSB > 0 ? LSB : 16];
+        };
+        Shared &sh;
+        const int tr0, tr1, grp, lane, lanebase;
+        bool lds_values;
+        __device__ Op(const SolveArgs &A, Shared &sh_, int row0, int row1)
+            : sh(sh_), tr0(row0 / B), tr1(row1 / B), grp(threadIdx.x / B), lane(threadIdx.x % B),
+              lanebase((threadIdx.x & 63) & ~(B - 1))
+        {
+            lds_values = stage_chunk<TPB>(A, tr0, tr1, TRW, sh.h, sh.t0, sh.slab, LSB);
+        }
+        // the layout as the SpMV and the passes read it
+        template <bool LDSV> __device__ DevL layout(const SolveArgs &A) const
+        {
+            DevL L = A.L;
+            if constexpr (LDSV) L.blob = sh.slab;
+            return L;
+        }
+        // y of the thread's rows, handed to body(i, y) for i ascending;
+        // with four-byte indices UQL4 and UQ64 quads of a row are in flight.
+        template <bool LDSV, int UQL4, int UQ64, typename F>
+        __device__ __forceinline__ void product(const SolveArgs &A, int, const double *g64, const float *g32,
+                                                F &&body) const
+        {
+            const DevL L = layout<LDSV>(A);
+#pragma unroll 1
+            for (int i0 = 0; i0 < RPT; i0 += NR) {
+                double w[NR];
+                tile_rows_spmv<B, IW, NR, GPB, UQL4, UQ64, CM>(L, sh.h, sh.t0, i0 * GPB + grp, tr0 + i0 * GPB + grp,
+                                                               lane, lanebase, g64, g32, w);
+#pragma unroll
+                for (int k = 0; k < NR; k++)
+                    if (tr0 + (i0 + k) * GPB + grp < tr1) body(i0 + k, w[k]);
+            }
+        }
+        // FP64-accumulated product of row slot i (the true-residual passes)
+        template <bool LDSV, int NV>
+        __device__ __forceinline__ void pass_row(const SolveArgs &A, int i, size_t, const double *const (&g)[NV],
+                                                 double (&acc)[NV]) const
+        {
+            const int q = i * GPB + grp, tr = tr0 + q;
+            if (A.use64) {
+                tile_row_spmv_f64_c<B, IW, NV>(A.L64, row_ctx<B, IW>(A.L64, tr, lane), lane, lanebase, g, acc);
+            } else {
+                const DevL L = layout<LDSV>(A);
+                tile_row_spmv_f64_c<B, IW, NV>(
+                    L, row_ctx_from<B, IW>(L, tr, sh.t0[q], sh.t0[q + 1] - sh.t0[q], sh.h[2 * q], sh.h[2 * q + 1], lane),
+                    lane, lanebase, g, acc);
+            }
+        }
+    };
+};
+
 // CG (Hestenes-Stiefel with s = A p carried by recurrence): registers hold
 // x and p of the thread's rows, LDS holds r and s.  Per iteration: [r
 // published, (r, r) reduced] -> convergence test -> w = A r, s = w + beta s,
@@ -364,54 +450,49 @@ __device__ bool stage_chunk(const SolveArgs &A, int tr0, int tr1, int TRW, int4 
 // rather than recurred (Chronopoulos-Gear's (A r, r) - beta (r, r) / alpha
 // form), which holds after a residual replacement that keeps the direction
 // and, with lossy tiles, halves the iterations on rough coefficients.
-template <int B, int IW, int TPB, int RPT, int CM = CM_ALL>
+template <class M, int TPB, int RPT>
 __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
 {
-    __shared__ double s_r[RPT * TPB];
+    // beyond X_REGS_ROWS rows per thread x stays in the caller's buffer
+    constexpr bool r_regs = M::r_regs, x_hbm = RPT > X_REGS_ROWS;
+    using Op = typename M::template Op<TPB, RPT, r_regs ? 1 : 2, 2 + 2 * r_regs + 2 * !x_hbm>;
+    __shared__ double s_r[r_regs ? 1 : RPT * TPB];
     __shared__ double s_s[RPT * TPB];
     __shared__ double s_red[(TPB / 64) * 4];
     __shared__ double s_bc[4];
     __shared__ int s_flag;
+    __shared__ typename Op::Shared s_op;
     Reducer<TPB, 4> R{s_red, s_bc, &s_flag};
-    constexpr int GPB = TPB / B, NR = spmv_rows(RPT, IW);
     const int tid = threadIdx.x;
     const int chunk = xcd_chunk(blockIdx.x, gridDim.x);
-    const int grp = tid / B, lane = tid % B, lanebase = (tid & 63) & ~(B - 1);
-    const int tr0 = chunk * A.trw, tr1 = min(A.tilem, tr0 + A.trw);
-    double xr[RPT], pr[RPT];
-    // headers of the block's tile rows, loaded once: the per-iteration SpMV
-    // then issues the tile-column word and the slab loads together
-    constexpr int TRW = RPT * GPB;
-    __shared__ int4 s_h[2 * TRW];
-    __shared__ int s_t0[TRW + 1];
-    // small chunks keep their slabs in LDS too
-    constexpr int LSB = lds_slab_bytes(RPT);
-    __shared__ __align__(16) uint8_t s_slab[LSB > 0 ? LSB : 16];
-    const bool lds_s = stage_chunk<TPB>(A, tr0, tr1, TRW, s_h, s_t0, s_slab, LSB);
+    const int row0 = chunk * A.crows, row1 = min(A.nrows, row0 + A.crows);
+    double xr[x_hbm ? 1 : RPT], pr[RPT], rr[r_regs ? RPT : 1];
+    auto r_at = [&](int i) -> double & {
+        if constexpr (r_regs) return rr[i];
+        else return s_r[i * TPB + tid];
+    };
+    const Op op(A, s_op, row0, row1);
     // one workgroup with the whole gathered vector in LDS (up to LDS_GATHER
     // rows): the SpMV reads published entries there, with no global stores
     // to drain and no cache round trips
     constexpr int LG = RPT <= 4 ? LDS_GATHER : 1;
     __shared__ double s_g64[LG];
     __shared__ float s_g32[LG];
-    const bool lds_g = RPT <= 4 && A.G == 1 && (long long)A.tilem * B <= LDS_GATHER;
+    const bool lds_g = RPT <= 4 && A.G == 1 && A.nrows <= LDS_GATHER;
     if (lds_g)
         for (int i = tid; i < LG; i += TPB) {
             s_g64[i] = 0.0;
             s_g32[i] = 0.0f;
         }
     __syncthreads();
-    int rbase = tr0 * B + tid;  // row of step i is rbase + i * TPB
-    auto tile_row = [&](int i) { return tr0 + i * GPB + grp; };
+    int rbase = row0 + tid;  // row of step i is rbase + i * TPB
+    auto live = [&](int i) { return rbase + i * TPB < row1; };
     auto row_of = [&](int i) { return (size_t)(rbase + i * TPB); };
     // the solve, with the gathered vector and the slabs each in LDS or in
     // global memory (up to four inlined copies, each with its address spaces
     // known to the compiler)
     auto solve = [&](double *g64, float *g32, auto lds_tag, auto slab_tag) {
-        constexpr bool lds = decltype(lds_tag)::value;
-        // the layout as the SpMV and the passes read it: slabs in LDS or HBM
-        DevL Lw = A.L;
-        if constexpr (decltype(slab_tag)::value) Lw.blob = s_slab;
+        constexpr bool lds = decltype(lds_tag)::value, ldsv = decltype(slab_tag)::value;
         auto publish = [&](size_t row, double v) {
             if (lds) {
                 if (A.has64) g64[row] = v;
@@ -422,9 +503,11 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
             }
         };
         auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
+            if constexpr (!x_hbm) {
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) A.x[row_of(i)] = xr[i];
+                for (int i = 0; i < RPT; i++)
+                    if (live(i)) A.x[row_of(i)] = xr[i];
+            }
             if (blockIdx.x == 0 && tid == 0) {
                 A.ctl[1] = status;
                 A.ctl[2] = iter;
@@ -437,13 +520,15 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
         double v1[1] = {0.0};
     #pragma clang loop unroll(full)
         for (int i = 0; i < RPT; i++) {
-            xr[i] = pr[i] = 0.0;
-            s_r[i * TPB + tid] = 0.0;
+            if constexpr (!x_hbm) xr[i] = 0.0;
+            pr[i] = 0.0;
+            r_at(i) = 0.0;
             s_s[i * TPB + tid] = 0.0;
-            if (tile_row(i) < tr1) {
+            if (live(i)) {
                 const size_t row = row_of(i);
                 const double bv = A.b[row];
-                s_r[i * TPB + tid] = bv;
+                r_at(i) = bv;
+                if constexpr (x_hbm) A.x[row] = 0.0;
                 publish(row, bv);
                 v1[0] += bv * bv;
             }
@@ -467,32 +552,35 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 // true residual b - A x and s = A p in one FP64-accumulated pass
     #pragma clang loop unroll(full)
                 for (int i = 0; i < RPT; i++)
-                    if (tile_row(i) < tr1) {
-                        st_agent(A.h64 + row_of(i), xr[i]);
+                    if (live(i)) {
+                        st_agent(A.h64 + row_of(i), x_hbm ? A.x[row_of(i)] : xr[x_hbm ? 0 : i]);
                         st_agent(A.q64 + row_of(i), pr[i]);
                     }
                 if (!R.barrier(A)) return;
                 double t1[1] = {0.0};
     #pragma unroll 1
-                for (int i = 0; i < RPT; i++) {
-                    const int tr = tile_row(i);
-                    if (tr < tr1) {
+                for (int i = 0; i < RPT; i++)
+                    if (live(i)) {
                         const double *g[2] = {A.h64, A.q64};
                         double acc[2] = {0.0, 0.0};
-                        const int q = i * GPB + grp;
-                        if (A.use64)
-                            tile_row_spmv_f64_c<B, IW, 2>(A.L64, row_ctx<B, IW>(A.L64, tr, lane), lane, lanebase, g, acc);
-                        else
-                            tile_row_spmv_f64_c<B, IW, 2>(
-                                Lw, row_ctx_from<B, IW>(Lw, tr, s_t0[q], s_t0[q + 1] - s_t0[q], s_h[2 * q], s_h[2 * q + 1], lane),
-                                lane, lanebase, g, acc);
-                        const size_t row = (size_t)tr * B + lane;
+                        const size_t row = row_of(i);
+                        op.template pass_row<ldsv, 2>(A, i, row, g, acc);
                         const double rv = A.b[row] - acc[0];
-                        s_r[i * TPB + tid] = rv;
                         s_s[i * TPB + tid] = acc[1];
                         publish(row, rv);
+                        // registers take no running index: the FP64 copy of
+                        // the published vector hands rv over
+                        if constexpr (r_regs) {
+                            if (lds || !A.has64) A.g64[row] = rv;
+                        } else {
+                            r_at(i) = rv;
+                        }
                         t1[0] += rv * rv;
                     }
+                if constexpr (r_regs) {
+    #pragma clang loop unroll(full)
+                    for (int i = 0; i < RPT; i++)
+                        if (live(i)) r_at(i) = A.g64[row_of(i)];
                 }
                 if (!R.allreduce(A, t1, true)) return;
                 clk.lap(4);
@@ -516,28 +604,20 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
             restart = false;
             const double beta = fresh ? 0.0 : gamma / gprev;
             // w = A r; s = w + beta s
-    #pragma unroll 1
-            for (int i0 = 0; i0 < RPT; i0 += NR) {
-                double w[NR];
-                // four-byte indices: four quads of a row in flight up to 8 rows per
-                // thread (at 16 the registers spill; BiCGSTAB's allow four only
-                // for FP64)
-                tile_rows_spmv<B, IW, NR, GPB, RPT <= 8 ? 4 : 2, RPT <= 8 ? 4 : 1, CM>(
-                    Lw, s_h, s_t0, i0 * GPB + grp, tile_row(i0), lane, lanebase, g64, g32, w);
-    #pragma unroll
-                for (int k = 0; k < NR; k++) {
-                    const int i = i0 + k;
-                    if (tile_row(i) < tr1) s_s[i * TPB + tid] = w[k] + beta * s_s[i * TPB + tid];
-                }
-            }
+            // (four-byte indices: four quads of a row in flight up to 8 rows
+            // per thread -- at 16 the registers spill; BiCGSTAB's allow four
+            // only for FP64)
+            op.template product<ldsv, RPT <= 8 ? 4 : 2, RPT <= 8 ? 4 : 1>(
+                A, rbase, g64, g32,
+                [&](int i, double w) { s_s[i * TPB + tid] = w + beta * s_s[i * TPB + tid]; });
             // p = r + beta p; (p, s)
             double red[1] = {0.0};
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    pr[i] = s_r[i * TPB + tid] + beta * pr[i];
-                    red[0] += pr[i] * s_s[i * TPB + tid];
-                }
+            for (int i = 0; i < RPT; i++) {
+                pr[i] = r_at(i) + beta * pr[i];
+                red[0] += pr[i] * s_s[i * TPB + tid];
+                if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
             clk.lap(0);
             if (!R.allreduce(A, red, false)) return;
             clk.lap(1);
@@ -551,36 +631,43 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 continue;
             }
             const double alpha = gamma / denom;
-    #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) xr[i] = xr[i] + alpha * pr[i];
             double g1[1] = {0.0};
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    const double rv = s_r[i * TPB + tid] - alpha * s_s[i * TPB + tid];
-                    s_r[i * TPB + tid] = rv;
-                    publish(row_of(i), rv);
-                    g1[0] += rv * rv;
-                }
+            for (int i = 0; i < RPT; i++) {
+                if constexpr (!x_hbm) xr[i] = xr[i] + alpha * pr[i];
+                const double rv = r_at(i) - alpha * s_s[i * TPB + tid];
+                r_at(i) = rv;
+                if (live(i)) publish(row_of(i), rv);
+                g1[0] += rv * rv;
+                if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
             gprev = gamma;
             ++iter;
             clk.lap(2);
-            if (!R.allreduce(A, g1, true)) return;
+            auto update_x = [&] {
+                if constexpr (x_hbm) {
+    #pragma clang loop unroll(full)
+                    for (int i = 0; i < RPT; i++) {
+                        if (live(i)) A.x[row_of(i)] += alpha * pr[i];
+                        if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            };
+            if (!R.allreduce(A, g1, true, update_x)) return;
             clk.lap(3);
             gamma = g1[0];
         }
     };
-    if constexpr (LSB > 0) {
-        if (lds_g) {
-            if (lds_s)
-                solve(s_g64, s_g32, std::true_type{}, std::true_type{});
-            else
-                solve(s_g64, s_g32, std::true_type{}, std::false_type{});
-            return;
+    if constexpr (RPT <= 4) {
+        if constexpr (M::lds_tags) {
+            if (op.lds_values) {
+                if (lds_g) solve(s_g64, s_g32, std::true_type{}, std::true_type{});
+                else solve(A.g64, A.g32, std::false_type{}, std::true_type{});
+                return;
+            }
         }
-        if (lds_s) {
-            solve(A.g64, A.g32, std::false_type{}, std::true_type{});
+        if (lds_g) {
+            solve(s_g64, s_g32, std::true_type{}, std::false_type{});
             return;
         }
     }
@@ -603,54 +690,43 @@ __device__ __forceinline__ void next_rho_g2(const double (&d)[5], double omega, 
 // omega^2 (t, t) -- the values of (r^, r) and (r, r) in exact arithmetic --
 // without a reduction of their own; s and p are published with neighbour
 // waits.
-template <int B, int IW, int TPB, int RPT, int CM = CM_ALL>
+template <class M, int TPB, int RPT>
 __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
 {
+    using Op = typename M::template Op<TPB, RPT, 2, 10>;
     __shared__ double s_v[RPT * TPB];
     __shared__ double s_t[RPT * TPB];
     __shared__ double s_red[(TPB / 64) * 5];
     __shared__ double s_bc[5];
     __shared__ int s_flag;
+    __shared__ typename Op::Shared s_op;
     Reducer<TPB, 5> R{s_red, s_bc, &s_flag};
-    constexpr int GPB = TPB / B, NR = spmv_rows(RPT, IW);
     const int tid = threadIdx.x;
     const int chunk = xcd_chunk(blockIdx.x, gridDim.x);
-    const int grp = tid / B, lane = tid % B, lanebase = (tid & 63) & ~(B - 1);
-    const int tr0 = chunk * A.trw, tr1 = min(A.tilem, tr0 + A.trw);
+    const int row0 = chunk * A.crows, row1 = min(A.nrows, row0 + A.crows);
     double xr[RPT], rr[RPT], rh[RPT], pr[RPT], sr[RPT];
-    // headers of the block's tile rows, loaded once: the per-iteration SpMV
-    // then issues the tile-column word and the slab loads together
-    constexpr int TRW = RPT * GPB;
-    __shared__ int4 s_h[2 * TRW];
-    __shared__ int s_t0[TRW + 1];
-    // small chunks keep their slabs in LDS too
-    constexpr int LSB = lds_slab_bytes(RPT);
-    __shared__ __align__(16) uint8_t s_slab[LSB > 0 ? LSB : 16];
-    const bool lds_s = stage_chunk<TPB>(A, tr0, tr1, TRW, s_h, s_t0, s_slab, LSB);
+    const Op op(A, s_op, row0, row1);
     // one workgroup with the whole gathered vector in LDS (up to LDS_GATHER
     // rows): the SpMV reads published entries there, with no global stores
     // to drain and no cache round trips
     constexpr int LG = RPT <= 4 ? LDS_GATHER : 1;
     __shared__ double s_g64[LG];
     __shared__ float s_g32[LG];
-    const bool lds_g = RPT <= 4 && A.G == 1 && (long long)A.tilem * B <= LDS_GATHER;
+    const bool lds_g = RPT <= 4 && A.G == 1 && A.nrows <= LDS_GATHER;
     if (lds_g)
         for (int i = tid; i < LG; i += TPB) {
             s_g64[i] = 0.0;
             s_g32[i] = 0.0f;
         }
     __syncthreads();
-    int rbase = tr0 * B + tid;  // row of step i is rbase + i * TPB
-    auto tile_row = [&](int i) { return tr0 + i * GPB + grp; };
+    int rbase = row0 + tid;  // row of step i is rbase + i * TPB
+    auto live = [&](int i) { return rbase + i * TPB < row1; };
     auto row_of = [&](int i) { return (size_t)(rbase + i * TPB); };
     // the solve, with the gathered vector and the slabs each in LDS or in
     // global memory (up to four inlined copies, each with its address spaces
     // known to the compiler)
     auto solve = [&](double *g64, float *g32, auto lds_tag, auto slab_tag) {
-        constexpr bool lds = decltype(lds_tag)::value;
-        // the layout as the SpMV and the passes read it: slabs in LDS or HBM
-        DevL Lw = A.L;
-        if constexpr (decltype(slab_tag)::value) Lw.blob = s_slab;
+        constexpr bool lds = decltype(lds_tag)::value, ldsv = decltype(slab_tag)::value;
         auto publish = [&](size_t row, double v) {
             if (lds) {
                 if (A.has64) g64[row] = v;
@@ -663,7 +739,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
         auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) A.x[row_of(i)] = xr[i];
+                if (live(i)) A.x[row_of(i)] = xr[i];
             if (blockIdx.x == 0 && tid == 0) {
                 A.ctl[1] = status;
                 A.ctl[2] = iter;
@@ -673,23 +749,16 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             }
         };
         auto spmv_into = [&](double *dst) {
-    #pragma unroll 1
-            for (int i0 = 0; i0 < RPT; i0 += NR) {
-                double w[NR];
-                tile_rows_spmv<B, IW, NR, GPB, 2, 4, CM>(Lw, s_h, s_t0, i0 * GPB + grp, tile_row(i0), lane, lanebase,
-                                                         g64, g32, w);
-    #pragma unroll
-                for (int k = 0; k < NR; k++)
-                    if (tile_row(i0 + k) < tr1) dst[(i0 + k) * TPB + tid] = w[k];
-            }
+            op.template product<ldsv, 2, 4>(A, rbase, g64, g32, [&](int i, double w) { dst[i * TPB + tid] = w; });
         };
 
         double v1[1] = {0.0};
     #pragma clang loop unroll(full)
         for (int i = 0; i < RPT; i++) {
             xr[i] = rr[i] = rh[i] = pr[i] = sr[i] = 0.0;
-            s_v[i * TPB + tid] = 0.0;
-            if (tile_row(i) < tr1) {
+            // zeros in the rows beyond the chunk, which the sums below include
+            s_v[i * TPB + tid] = s_t[i * TPB + tid] = 0.0;
+            if (live(i)) {
                 const size_t row = row_of(i);
                 rr[i] = rh[i] = pr[i] = A.b[row];
                 publish(row, pr[i]);
@@ -711,18 +780,16 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             clk.lap(0);
             double a1[1] = {0.0};
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) a1[0] += rh[i] * s_v[i * TPB + tid];
+            for (int i = 0; i < RPT; i++) a1[0] += rh[i] * s_v[i * TPB + tid];
             if (!R.allreduce(A, a1, false)) return;
             clk.lap(1);
             if (!(a1[0] != 0.0) || !isfinite(a1[0])) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, -1.0); return; }
             const double alpha = rho / a1[0];
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    sr[i] = rr[i] - alpha * s_v[i * TPB + tid];
-                    publish(row_of(i), sr[i]);
-                }
+            for (int i = 0; i < RPT; i++) {
+                sr[i] = rr[i] - alpha * s_v[i * TPB + tid];
+                if (live(i)) publish(row_of(i), sr[i]);
+            }
             clk.lap(2);
             if (!R.published(A, chunk)) return;
             clk.lap(3);
@@ -730,24 +797,22 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             clk.lap(0);
             double a2[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    const double t = s_t[i * TPB + tid];
-                    a2[0] += t * sr[i];
-                    a2[1] += t * t;
-                    a2[2] += rh[i] * sr[i];
-                    a2[3] += rh[i] * t;
-                    a2[4] += sr[i] * sr[i];
-                }
+            for (int i = 0; i < RPT; i++) {
+                const double t = s_t[i * TPB + tid];
+                a2[0] += t * sr[i];
+                a2[1] += t * t;
+                a2[2] += rh[i] * sr[i];
+                a2[3] += rh[i] * t;
+                a2[4] += sr[i] * sr[i];
+            }
             if (!R.allreduce(A, a2, false)) return;
             clk.lap(1);
             const double omega = a2[1] > 0.0 ? a2[0] / a2[1] : 0.0;
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    xr[i] = xr[i] + alpha * pr[i] + omega * sr[i];
-                    rr[i] = sr[i] - omega * s_t[i * TPB + tid];
-                }
+            for (int i = 0; i < RPT; i++) {
+                xr[i] = xr[i] + alpha * pr[i] + omega * sr[i];
+                rr[i] = sr[i] - omega * s_t[i * TPB + tid];
+            }
             double rho_new, g2;
             next_rho_g2(a2, omega, rho_new, g2);
             ++iter;
@@ -757,28 +822,21 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             if (conv || due) {
     #pragma clang loop unroll(full)
                 for (int i = 0; i < RPT; i++)
-                    if (tile_row(i) < tr1) st_agent(A.h64 + row_of(i), xr[i]);
+                    if (live(i)) st_agent(A.h64 + row_of(i), xr[i]);
                 if (!R.barrier(A)) return;
     #pragma unroll 1
-                for (int i = 0; i < RPT; i++) {
-                    const int tr = tile_row(i);
-                    if (tr < tr1) {
+                for (int i = 0; i < RPT; i++)
+                    if (live(i)) {
                         const double *g[1] = {A.h64};
                         double acc[1] = {0.0};
-                        const int q = i * GPB + grp;
-                        if (A.use64)
-                            tile_row_spmv_f64_c<B, IW, 1>(A.L64, row_ctx<B, IW>(A.L64, tr, lane), lane, lanebase, g, acc);
-                        else
-                            tile_row_spmv_f64_c<B, IW, 1>(
-                                Lw, row_ctx_from<B, IW>(Lw, tr, s_t0[q], s_t0[q + 1] - s_t0[q], s_h[2 * q], s_h[2 * q + 1], lane),
-                                lane, lanebase, g, acc);
-                        s_t[i * TPB + tid] = A.b[(size_t)tr * B + lane] - acc[0];
+                        const size_t row = row_of(i);
+                        op.template pass_row<ldsv, 1>(A, i, row, g, acc);
+                        s_t[i * TPB + tid] = A.b[row] - acc[0];
                     }
-                }
                 double t2[2] = {0.0, 0.0};
     #pragma clang loop unroll(full)
                 for (int i = 0; i < RPT; i++)
-                    if (tile_row(i) < tr1) {
+                    if (live(i)) {
                         rr[i] = s_t[i * TPB + tid];
                         t2[0] += rr[i] * rr[i];
                         t2[1] += rr[i] * rh[i];
@@ -799,27 +857,26 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             const double beta = restart ? 0.0 : (rho_new / rho) * (alpha / omega);
             restart = false;
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++)
-                if (tile_row(i) < tr1) {
-                    pr[i] = rr[i] + beta * (pr[i] - omega * s_v[i * TPB + tid]);
-                    publish(row_of(i), pr[i]);
-                }
+            for (int i = 0; i < RPT; i++) {
+                pr[i] = rr[i] + beta * (pr[i] - omega * s_v[i * TPB + tid]);
+                if (live(i)) publish(row_of(i), pr[i]);
+            }
             rho = rho_new;
             clk.lap(2);
             if (!R.published(A, chunk)) return;
             clk.lap(3);
         }
     };
-    if constexpr (LSB > 0) {
-        if (lds_g) {
-            if (lds_s)
-                solve(s_g64, s_g32, std::true_type{}, std::true_type{});
-            else
-                solve(s_g64, s_g32, std::true_type{}, std::false_type{});
-            return;
+    if constexpr (RPT <= 4) {
+        if constexpr (M::lds_tags) {
+            if (op.lds_values) {
+                if (lds_g) solve(s_g64, s_g32, std::true_type{}, std::true_type{});
+                else solve(A.g64, A.g32, std::false_type{}, std::true_type{});
+                return;
+            }
         }
-        if (lds_s) {
-            solve(A.g64, A.g32, std::false_type{}, std::true_type{});
+        if (lds_g) {
+            solve(s_g64, s_g32, std::true_type{}, std::false_type{});
             return;
         }
     }
@@ -1191,6 +1248,7 @@ struct KernelChoice {
     int tpb = 0, rpt = 0;
     int streamed = 0;  // 1: vectors in HBM (k_cg_st / k_bicgstab_st), rpt = 0
     int acc64 = 0;     // 1: built with CM_ACC64 (publishes the FP64 vector only)
+    int stencil = 0;   // 1: on stencil planes
 };
 
 constexpr int ST_TPB = 512;
@@ -1207,20 +1265,20 @@ KernelChoice pick_kernel(int method, long long rows_per_wg, bool stream)
     const int q = (int)((rows_per_wg + 511) / 512);
     if (stream) {
     } else if (method == MF_CG) {
-        if (q <= 1) k = {k_cg<B, IW, 512, 1>, 512, 1};
-        else if (q <= 2) k = {k_cg<B, IW, 512, 2>, 512, 2};
-        else if (q <= 4) k = {k_cg<B, IW, 512, 4>, 512, 4};
-        else if (q <= 8) k = {k_cg<B, IW, 512, 8>, 512, 8};
+        if (q <= 1) k = {k_cg<Slabs<B, IW>, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_cg<Slabs<B, IW>, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_cg<Slabs<B, IW>, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_cg<Slabs<B, IW>, 512, 8>, 512, 8};
         // 16 rows per thread: r, s and the headers of 1024 tile rows of 8
         // rows exceed the 160 KB of LDS, so 8-row tiles stop at 8
         else if constexpr (B >= 16) {
-            if (q <= 16) k = {k_cg<B, IW, 512, 16>, 512, 16};
+            if (q <= 16) k = {k_cg<Slabs<B, IW>, 512, 16>, 512, 16};
         }
     } else {
-        if (q <= 1) k = {k_bicgstab<B, IW, 512, 1>, 512, 1};
-        else if (q <= 2) k = {k_bicgstab<B, IW, 512, 2>, 512, 2};
-        else if (q <= 4) k = {k_bicgstab<B, IW, 512, 4>, 512, 4};
-        else if (q <= 8) k = {k_bicgstab<B, IW, 512, 8>, 512, 8};
+        if (q <= 1) k = {k_bicgstab<Slabs<B, IW>, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_bicgstab<Slabs<B, IW>, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_bicgstab<Slabs<B, IW>, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_bicgstab<Slabs<B, IW>, 512, 8>, 512, 8};
     }
     if (!k.fn)
         k = {method == MF_CG ? k_cg_st<B, IW, ST_TPB> : k_bicgstab_st<B, IW, ST_TPB>, ST_TPB, 0, 1};
@@ -1239,14 +1297,14 @@ KernelChoice pick_kernel_cm(int method, long long rows_per_wg)
     const int q = (int)((rows_per_wg + 511) / 512);
     if (q <= 2) return k;
     if (method == MF_CG) {
-        if (q <= 4) k = {k_cg<B, IW, 512, 4, CM>, 512, 4};
-        else if (q <= 8) k = {k_cg<B, IW, 512, 8, CM>, 512, 8};
+        if (q <= 4) k = {k_cg<Slabs<B, IW, CM>, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_cg<Slabs<B, IW, CM>, 512, 8>, 512, 8};
         else if constexpr (B >= 16) {
-            if (q <= 16) k = {k_cg<B, IW, 512, 16, CM>, 512, 16};
+            if (q <= 16) k = {k_cg<Slabs<B, IW, CM>, 512, 16>, 512, 16};
         }
     } else {
-        if (q <= 4) k = {k_bicgstab<B, IW, 512, 4, CM>, 512, 4};
-        else if (q <= 8) k = {k_bicgstab<B, IW, 512, 8, CM>, 512, 8};
+        if (q <= 4) k = {k_bicgstab<Slabs<B, IW, CM>, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_bicgstab<Slabs<B, IW, CM>, 512, 8>, 512, 8};
     }
     return k;
 }
@@ -1271,13 +1329,13 @@ KernelChoice pick_kernel_acc64(int method, long long rows_per_wg, int G)
     const int q = (int)((rows_per_wg + 511) / 512);
     if (q > 1 && G != 1) return k;
     if (method == MF_CG) {
-        if (q <= 1) k = {k_cg<B, IW, 512, 1, CMA>, 512, 1};
-        else if (q <= 2) k = {k_cg<B, IW, 512, 2, CMA>, 512, 2};
-        else if (q <= 4) k = {k_cg<B, IW, 512, 4, CMA>, 512, 4};
+        if (q <= 1) k = {k_cg<Slabs<B, IW, CMA>, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_cg<Slabs<B, IW, CMA>, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_cg<Slabs<B, IW, CMA>, 512, 4>, 512, 4};
     } else {
-        if (q <= 1) k = {k_bicgstab<B, IW, 512, 1, CMA>, 512, 1};
-        else if (q <= 2) k = {k_bicgstab<B, IW, 512, 2, CMA>, 512, 2};
-        else if (q <= 4) k = {k_bicgstab<B, IW, 512, 4, CMA>, 512, 4};
+        if (q <= 1) k = {k_bicgstab<Slabs<B, IW, CMA>, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_bicgstab<Slabs<B, IW, CMA>, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_bicgstab<Slabs<B, IW, CMA>, 512, 4>, 512, 4};
     }
     k.acc64 = k.fn ? 1 : 0;
     return k;
@@ -1289,6 +1347,61 @@ template <int B> KernelChoice pick_tile_acc64(int iw, int method, long long rows
            : iw == 2 ? pick_kernel_acc64<B, 2>(method, rows_per_wg, G)
                      : pick_kernel_acc64<B, 4>(method, rows_per_wg, G);
 }
+
+// Resident kernels on the stencil planes of class cls (a64: low-precision
+// values summed in FP64, see pick_kernel_acc64).  Rows per thread go up to 28
+// for CG: x, p and r of a row in registers, s in LDS.
+template <class M> KernelChoice pick_stencil_kernel(int method, long long rows_per_wg)
+{
+    KernelChoice k;
+    const int q = (int)((rows_per_wg + 511) / 512);
+    if (method == MF_CG) {
+        if (q <= 1) k = {k_cg<M, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_cg<M, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_cg<M, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_cg<M, 512, 8>, 512, 8};
+        else if (q <= 16) k = {k_cg<M, 512, 16>, 512, 16};
+        // beyond: x in HBM, so these count as streamed
+        else if (q <= 20) k = {k_cg<M, 512, 20>, 512, 20, 1};
+        else if (q <= 28) k = {k_cg<M, 512, 28>, 512, 28, 1};
+        else if (q <= 36) k = {k_cg<M, 512, 36>, 512, 36, 1};
+    } else {
+        if (q <= 1) k = {k_bicgstab<M, 512, 1>, 512, 1};
+        else if (q <= 2) k = {k_bicgstab<M, 512, 2>, 512, 2};
+        else if (q <= 4) k = {k_bicgstab<M, 512, 4>, 512, 4};
+        else if (q <= 8) k = {k_bicgstab<M, 512, 8>, 512, 8};
+    }
+    return k;
+}
+template <class M> KernelChoice pick_stencil_acc64(int method, long long rows_per_wg, int G)
+{
+    KernelChoice k;
+    const int q = (int)((rows_per_wg + 511) / 512);
+    if (q > 4 || (q > 1 && G != 1)) return k;
+    if (method == MF_CG) k = {q <= 1 ? k_cg<M, 512, 1> : q <= 2 ? k_cg<M, 512, 2> : k_cg<M, 512, 4>, 512, q <= 1 ? 1 : q <= 2 ? 2 : 4};
+    else k = {q <= 1 ? k_bicgstab<M, 512, 1> : q <= 2 ? k_bicgstab<M, 512, 2> : k_bicgstab<M, 512, 4>, 512, q <= 1 ? 1 : q <= 2 ? 2 : 4};
+    k.acc64 = 1;
+    return k;
+}
+template <int CLS> KernelChoice pick_stencil_class(int L, int method, long long rows_per_wg, int G)
+{
+    const int sw = plane_sw(L);
+    KernelChoice k;
+    if constexpr (CLS > 0) {
+        k = sw == 5   ? pick_stencil_acc64<Stencil<CLS, 5, true>>(method, rows_per_wg, G)
+            : sw == 7 ? pick_stencil_acc64<Stencil<CLS, 7, true>>(method, rows_per_wg, G)
+                      : pick_stencil_acc64<Stencil<CLS, 0, true>>(method, rows_per_wg, G);
+        if (k.fn) return k;
+    }
+    return sw == 5   ? pick_stencil_kernel<Stencil<CLS, 5, false>>(method, rows_per_wg)
+           : sw == 7 ? pick_stencil_kernel<Stencil<CLS, 7, false>>(method, rows_per_wg)
+                     : pick_stencil_kernel<Stencil<CLS, 0, false>>(method, rows_per_wg);
+}
+// one class each: solver_st64.hip, solver_st32.hip, solver_st16.hip, solver_st8.hip
+KernelChoice pick_stencil_f64(int L, int method, long long rows_per_wg, int G);
+KernelChoice pick_stencil_f32(int L, int method, long long rows_per_wg, int G);
+KernelChoice pick_stencil_f16(int L, int method, long long rows_per_wg, int G);
+KernelChoice pick_stencil_e4m3(int L, int method, long long rows_per_wg, int G);
 
 // tile sizes and class masks instantiated in their own translation units
 KernelChoice pick_b8(int iw, int method, long long rows_per_wg, bool stream);   // solver_b8.hip

@@ -121,6 +121,23 @@ static int layout_cm(const Layout &L)
     return !low ? CM_F64 : e4m3_only ? CM_E4M3 : !f64 ? CM_LOW : CM_ALL;
 }
 
+// The kernel on a layout's stencil planes (and, when the passes read the FP64
+// layout, on its planes too); none where they are missing or a workgroup's
+// rows exceed the resident kernels.
+static KernelChoice pick_stencil(mf_matrix m, const Layout &L, const Layout *L64, int method, long long rows_per_wg, int G)
+{
+    if (!L.planes || (L64 && L64 != &L && !L64->planes)) return KernelChoice{};
+    KernelChoice k;
+    switch (L.planes_cls) {
+    case 0: k = pick_stencil_f64(m->st_L, method, rows_per_wg, G); break;
+    case 1: k = pick_stencil_f32(m->st_L, method, rows_per_wg, G); break;
+    case 2: k = pick_stencil_f16(m->st_L, method, rows_per_wg, G); break;
+    case 3: k = pick_stencil_e4m3(m->st_L, method, rows_per_wg, G); break;
+    }
+    k.stencil = k.fn ? 1 : 0;
+    return k;
+}
+
 static KernelChoice pick(int B, int iw, int method, long long rows_per_wg, bool stream, int cm = CM_ALL, int G = 0)
 {
     if (B == 16 && !stream && cm != CM_F64) {
@@ -221,8 +238,9 @@ __global__ void k_chunk_deps(const int *__restrict__ tile_ptr, const int *__rest
 }
 
 // The neighbour lists of the grid (G chunks of trw tile rows), built once per
-// grid shape: the solvers wait only for these chunks after a publish when no
-// list is longer than one wave (64).
+// grid shape: BiCGSTAB waits only for these chunks after a publish when no list
+// is longer than one wave (64).
+static bool wants_deps(const mf_opts &o) { return o.method == MF_BICGSTAB && o.sync != MF_SYNC_GLOBAL; }
 static int ensure_deps(mf_matrix m, int G, int trw)
 {
     Workspace &w = m->ws;
@@ -327,9 +345,26 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     A.use64 = L64 && L64 != &L ? 1 : 0;
     A.L64 = A.use64 ? L64->view(m->d_tile_ptr) : A.L;
     if (A.use64 && L64->iw != L.iw) return fail(MF_E_FORMAT, "layouts with different index forms");
+    if (kc.stencil) {
+        auto view = [&](const Layout &Lv) {
+            Planes P{};
+            P.val = Lv.planes;
+            P.stride = (unsigned)((size_t)m->tilem * m->B);
+            P.L = m->st_L;
+            return P;
+        };
+        A.pl = view(L);
+        A.pl64 = A.use64 ? view(*L64) : A.pl;
+        A.off = m->d_st->off;
+    } else {
+        A.pl = A.pl64 = Planes{};
+        A.off = nullptr;
+    }
     A.tilem = m->tilem;
     A.G = G;
     A.trw = trw;
+    A.nrows = m->tilem * m->B;
+    A.crows = trw * m->B;
     A.b = d_b;
     A.x = d_x;
     A.g64 = w.g64;
@@ -351,10 +386,10 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     A.flags = w.flags;
     // BiCGSTAB's syncs after publishing p and s carry no reduction: they can
     // be neighbour waits (CG's publish sync also reduces (r, r))
-    A.nbr = method == MF_BICGSTAB && o.sync != MF_SYNC_GLOBAL && w.flags && w.dep_max >= 0 && w.dep_max <= 64 ? 1 : 0;
-    A.vec = kc.streamed ? w.vec : nullptr;
+    A.nbr = wants_deps(o) && w.flags && w.dep_max >= 0 && w.dep_max <= 64 ? 1 : 0;
+    A.vec = kc.streamed && !kc.stencil ? w.vec : nullptr;
     A.vstride = w.vstride;
-    if (kc.streamed && !w.vec) return fail(MF_E_ARG, "streamed kernel without its vectors");
+    if (kc.streamed && !kc.stencil && !w.vec) return fail(MF_E_ARG, "streamed kernel without its vectors");
     if (res) {
         res->sync_deps = A.nbr ? w.dep_max : -1;
         res->streamed = kc.streamed;
@@ -459,7 +494,8 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
 {
     int G = 1, trw = 1;
     solver_grid(m->tilem, m->B, o.grid, &G, &trw);
-    KernelChoice kc = pick(m->B, L.iw, method, (long long)trw * m->B, false, layout_cm(L), G);
+    KernelChoice kc = pick_stencil(m, L, L64, method, (long long)trw * m->B, G);
+    if (!kc.fn) kc = pick(m->B, L.iw, method, (long long)trw * m->B, false, layout_cm(L), G);
     if (!kc.fn) return fail(MF_E_UNSUPPORTED, "no persistent kernel for this tile size and index form");
     // streaming the vectors of a system whose rows fit on chip is switched
     // off: two runs that forced it on small grids ended with a GPU fault
@@ -470,12 +506,14 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
         return fail(MF_E_UNSUPPORTED, "vectors on chip: the system exceeds register/LDS residency at this grid");
     int rc = ensure_ws(m, G);
     if (rc) return rc;
-    if (kc.streamed) {
+    if (kc.streamed && !kc.stencil) {
         rc = ensure_vec(m, stream_vectors(method));
         if (rc) return rc;
     }
-    rc = ensure_deps(m, G, trw);
-    if (rc) return rc;
+    if (wants_deps(o)) {
+        rc = ensure_deps(m, G, trw);
+        if (rc) return rc;
+    }
     const Workspace &ws = m->ws;
     WsView w;
     w.g64 = ws.g64;
@@ -485,10 +523,12 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
     w.slots = ws.slots;
     w.ctl = ws.ctl;
     w.out = ws.out;
-    w.dep_ptr = ws.dep_ptr;
-    w.dep_idx = ws.dep_idx;
-    w.flags = ws.flags;
-    w.dep_max = ws.dep_max;
+    if (wants_deps(o)) {
+        w.dep_ptr = ws.dep_ptr;
+        w.dep_idx = ws.dep_idx;
+        w.flags = ws.flags;
+        w.dep_max = ws.dep_max;
+    }
     w.vec = ws.vec;
     w.vstride = (long long)ws.ncol;
     return launch_persistent(m, L, L64, method, d_b, d_x, tol, o, G, trw, kc, w, sync, res, grid_out, block_out,
@@ -541,15 +581,18 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
         rc = build_layout(m, m->Lmix, o.tau, o.allow_mask, want);
         if (rc) return rc;
     }
-    rep->ms_setup = now_ms() - t0;
     const Layout &L = mixed ? m->Lmix : m->L64;
     // lossless layout: the stored operator is A itself, so the kernel's own
     // true-residual test is final; a lossy layout either runs its passes on
     // the FP64 layout (ir_max_outer = 0) or is refined in FP64 around it
     const bool exact = !mixed || o.tau == 0.0;
+    rc = mixed ? ensure_planes(m, m->Lmix) : MF_OK;
+    if (!rc && (!mixed || !exact)) rc = ensure_planes(m, m->L64);
+    if (rc) return rc;
+    rep->ms_setup = now_ms() - t0;
     rc = ensure_ws(m, std::max(1, o.grid > 0 ? o.grid : device_cu_count()));
     if (rc) return rc;
-    {  // the grid's neighbour lists, outside the timed region
+    if (wants_deps(o)) {  // the grid's neighbour lists, outside the timed region
         int G0 = 1, trw0 = 1;
         solver_grid(m->tilem, m->B, o.grid, &G0, &trw0);
         rc = ensure_deps(m, G0, trw0);
@@ -725,7 +768,9 @@ static int noalloc_core(mf_matrix m, int dev, const double *d_b, double *d_x, co
     int G = 1, trw = 1;
     solver_grid(m->tilem, m->B, o.grid, &G, &trw);
     if (G > NA_MAX_G) return fail(MF_E_ARG, "allocation-free solve: more than 1024 workgroups");
-    const KernelChoice kc = pick(m->B, L.iw, o.method, (long long)trw * m->B, false, layout_cm(L), G);
+    const Layout *pass64 = exact ? nullptr : &m->L64;
+    KernelChoice kc = pick_stencil(m, L, pass64, o.method, (long long)trw * m->B, G);
+    if (!kc.fn) kc = pick(m->B, L.iw, o.method, (long long)trw * m->B, false, layout_cm(L), G);
     if (!kc.fn || kc.streamed)
         return fail(MF_E_UNSUPPORTED, "allocation-free solve: system beyond register/LDS residency at this grid");
     unsigned char *base = static_cast<unsigned char *>(g_scratch[dev]);
@@ -754,13 +799,14 @@ static int noalloc_core(mf_matrix m, int dev, const double *d_b, double *d_x, co
         MF_HIP(hipStreamSynchronize(st));
         return MF_OK;
     };
-    int rc = run(L, exact ? nullptr : &m->L64, kc);
+    int rc = run(L, pass64, kc);
     if (rc) return rc;
     int status = ctl[0] ? MF_E_TIMEOUT : ctl[1], iters = ctl[2], repl = ctl[3];
     // lossy tiles that failed: the same solve on the FP64 layout, as mf_solve_device
     if (!exact && (status == MF_E_DIVERGED || status == MF_E_BREAKDOWN || status == MF_E_NONFINITE ||
                    status == MF_E_MAXIT)) {
-        const KernelChoice k64 = pick(m->B, m->L64.iw, o.method, (long long)trw * m->B, false, layout_cm(m->L64), G);
+        KernelChoice k64 = pick_stencil(m, m->L64, nullptr, o.method, (long long)trw * m->B, G);
+        if (!k64.fn) k64 = pick(m->B, m->L64.iw, o.method, (long long)trw * m->B, false, layout_cm(m->L64), G);
         if (!k64.fn || k64.streamed) return fail(MF_E_UNSUPPORTED, "allocation-free solve: no FP64 kernel");
         rc = run(m->L64, nullptr, k64);
         if (rc) return rc;

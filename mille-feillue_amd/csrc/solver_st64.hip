@@ -1,0 +1,12 @@
+// Resident CG / BiCGSTAB kernels on stencil planes of FP64 values (instantiated
+// here so they compile in parallel).
+#include "persistent.h"
+
+namespace mf {
+
+KernelChoice pick_stencil_f64(int L, int method, long long rows_per_wg, int G)
+{
+    return pick_stencil_class<0>(L, method, rows_per_wg, G);
+}
+
+}  // namespace mf

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "mf_matrix.h"
+#include "stencil.h"
 
 namespace mf {
 
@@ -861,10 +862,143 @@ void Layout::release()
     if (trh) (void)hipFree(trh);
     if (stc) (void)hipFree(stc);
     if (blob) (void)hipFree(blob);
+    if (planes) (void)hipFree(planes);
+    planes = nullptr;
+    planes_cls = -1;
+    planes_tried = false;
     trh = nullptr;
     stc = nullptr;
     blob = nullptr;
     built = false;
+}
+
+// --------------------------------------------------------- stencil planes
+// key = (entries of the longest row << 32) | (its first occurrence, counted
+// from the end)
+__global__ __launch_bounds__(256) void k_longest_row(const int *__restrict__ rowptr, int rows, unsigned long long *key)
+{
+    __shared__ unsigned long long s_key;
+    if (threadIdx.x == 0) s_key = 0ull;
+    __syncthreads();
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r < rows)
+        atomicMax(&s_key, (unsigned long long)(rowptr[r + 1] - rowptr[r]) << 32 | (unsigned)(rows - 1 - r));
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(key, s_key);
+}
+
+// Table position of offset d (L: not in the table).
+__device__ __forceinline__ int offset_pos(const StencilTable *t, int d)
+{
+    int p = t->L;
+    for (int j = 0; j < t->L; j++)
+        if (t->off[j] == d) p = j;
+    return p;
+}
+
+// The longest row's offsets (one wave); bad when there are too many.
+__global__ __launch_bounds__(64) void k_stencil_table(const int *__restrict__ rowptr, const int *__restrict__ col,
+                                                      int rows, StencilTable *t)
+{
+    const unsigned long long key = t->key;
+    const int L = (int)(key >> 32), row = rows - 1 - (int)(unsigned)key, j = threadIdx.x;
+    if (j < STENCIL_MAX) t->off[j] = j < L && L <= STENCIL_MAX ? col[rowptr[row] + j] - row : 0;
+    if (j == 0) {
+        t->L = min(L, STENCIL_MAX);
+        t->bad = L < 1 || L > STENCIL_MAX;
+    }
+}
+
+// bad when some row's entries are not in strictly ascending column order or
+// have an offset outside the table
+__global__ __launch_bounds__(256) void k_stencil_check(const int *__restrict__ rowptr, const int *__restrict__ col,
+                                                       int rows, StencilTable *t)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= rows || t->bad) return;
+    int prev = -1;
+    for (int k = rowptr[r]; k < rowptr[r + 1]; k++) {
+        const int c = col[k];
+        if (c <= prev || offset_pos(t, c - r) == t->L) {
+            atomicOr(&t->bad, 1);
+            return;
+        }
+        prev = c;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_planes_pack(const int *__restrict__ rowptr, const int *__restrict__ col,
+                                                     const double *__restrict__ val, int rows,
+                                                     const StencilTable *__restrict__ t, int cls, size_t stride,
+                                                     uint8_t *__restrict__ out)
+{
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= rows) return;
+    const int L = t->L;
+    for (int k = rowptr[r]; k < rowptr[r + 1]; k++) {
+        uint8_t *p = out + plane_pos(cls, L, stride, (size_t)r, offset_pos(t, col[k] - r));
+        const double v = val[k];
+        switch (cls) {
+        case 0: *reinterpret_cast<double *>(p) = v; break;
+        case 1: *reinterpret_cast<float *>(p) = (float)v; break;
+        case 2: *reinterpret_cast<uint16_t *>(p) = f64_to_f16(v); break;
+        default: *p = f64_to_e4m3(v); break;
+        }
+    }
+}
+
+// Looks for the matrix's offset table: the longest row's offsets, when every
+// row is strictly ascending and draws from them.
+static int find_stencil(mf_matrix m)
+{
+    m->st_L = 0;
+    if (m->rowA != m->colA || !m->nnz || m->d_split) return MF_OK;
+    hipStream_t st = stream();
+    const unsigned nb = (unsigned)((m->rowA + 255) / 256);
+    if (!m->d_st) MF_HIP(hipMalloc((void **)&m->d_st, sizeof(StencilTable)));
+    MF_HIP(hipMemsetAsync(m->d_st, 0, sizeof(StencilTable), st));
+    k_longest_row<<<nb, 256, 0, st>>>(m->d_rowptr, m->rowA, &m->d_st->key);
+    k_stencil_table<<<1, 64, 0, st>>>(m->d_rowptr, m->d_col, m->rowA, m->d_st);
+    k_stencil_check<<<nb, 256, 0, st>>>(m->d_rowptr, m->d_col, m->rowA, m->d_st);
+    MF_HIP(hipGetLastError());
+    StencilTable t;
+    MF_HIP(hipMemcpyAsync(&t, m->d_st, sizeof(t), hipMemcpyDeviceToHost, st));
+    MF_HIP(hipStreamSynchronize(st));
+    if (!t.bad) m->st_L = t.L;
+    return MF_OK;
+}
+
+int ensure_planes(mf_matrix m, Layout &L)
+{
+    if (L.planes_tried || !L.built) return MF_OK;
+    L.planes_tried = true;
+    // one class, automatic index form
+    int cls = -1, classes = 0;
+    for (int code = 0; code < 5; code++)
+        if (L.tiles_per_code[code] > 0) {
+            cls = code_to_cls(code);
+            classes++;
+        }
+    if (classes != 1 || L.want_iw != 0 || L.split) return MF_OK;
+    if (m->st_L < 0) {
+        int rc = find_stencil(m);
+        if (rc) return rc;
+    }
+    if (!m->st_L) return MF_OK;
+    const size_t rows = (size_t)m->tilem * m->B;
+    const size_t bytes = rows * plane_row_bytes(cls, m->st_L);
+    // planes hold a value for every row and offset: worth it where that is
+    // little more than the slabs hold (boundary rows), not for tables that
+    // most rows use a few entries of
+    if (bytes > L.blob_bytes + L.blob_bytes / 4) return MF_OK;
+    hipStream_t st = stream();
+    MF_HIP(hipMalloc((void **)&L.planes, bytes));
+    MF_HIP(hipMemsetAsync(L.planes, 0, bytes, st));
+    k_planes_pack<<<(unsigned)((m->rowA + 255) / 256), 256, 0, st>>>(m->d_rowptr, m->d_col, m->d_val, m->rowA, m->d_st, cls,
+                                                                     rows, L.planes);
+    MF_HIP(hipGetLastError());
+    L.planes_cls = cls;
+    return MF_OK;
 }
 
 template <int B>

@@ -1,0 +1,96 @@
+"""Solves on stencil planes (matrices whose rows draw their entries from one
+short list of offsets) against the same solves on the slabs, bit for bit: an
+explicit index width keeps a solve on the slabs."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-10
+
+
+def _banded(n, offsets, rng, drop=0.0):
+    """Diagonally dominant symmetric matrix on the given positive offsets (and
+    their negatives); a share of the pairs is dropped."""
+    rows, cols, vals = [], [], []
+    diag = np.full(n, 0.25)
+    for d in offsets:
+        i = np.arange(n - d)
+        i = i[rng.random(len(i)) >= drop]
+        v = -rng.uniform(0.5, 1.5, len(i))
+        rows += [i, i + d]
+        cols += [i + d, i]
+        vals += [v, v]
+        np.subtract.at(diag, i, v)
+        np.subtract.at(diag, i + d, v)
+    rows.append(np.arange(n)), cols.append(np.arange(n)), vals.append(diag)
+    r, c, v = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int64)
+    np.add.at(rp, r + 1, 1)
+    return np.cumsum(rp).astype(np.int32), c[o].astype(np.int32), v[o]
+
+
+def _matrix(gpu, name):
+    rng = np.random.default_rng(5)
+    return {
+        "laplace2d_30x31": lambda: gpu.gen_laplace2d(30, 31),          # 5 offsets, one workgroup
+        "laplace2d_97x83": lambda: gpu.gen_laplace2d(97, 83),          # 5 offsets, ragged last tile row
+        "poisson3d_17x19x13": lambda: gpu.gen_poisson3d(17, 19, 13),   # 7 offsets
+        "poisson3d_33x31x29": lambda: gpu.gen_poisson3d(33, 31, 29),
+        "convdiff_14": lambda: gpu.gen_convdiff3d(14, 10.0, 1.0, 0),   # 27 offsets: quads
+        "convdiff_21": lambda: gpu.gen_convdiff3d(21, 10.0, 1.0, 0),
+        "lognormal_3d": lambda: gpu.gen_stencil_lognormal(3, 9000, 0.5, 3),
+        "band_3": lambda: _banded(1000, (1,), rng),                    # one quad, padded
+        "band_9": lambda: _banded(5003, (1, 7, 40, 41), rng),          # three quads, odd size
+        "band_31": lambda: _banded(4099, tuple(range(1, 16)), rng, 0.1),
+    }[name]()
+
+
+CASES = [("laplace2d_30x31", 0), ("laplace2d_97x83", 0), ("laplace2d_97x83", 1), ("poisson3d_17x19x13", 0),
+         ("poisson3d_33x31x29", 0), ("poisson3d_33x31x29", 3), ("convdiff_14", 0), ("convdiff_14", 2), ("convdiff_21", 0),
+         ("lognormal_3d", 0), ("lognormal_3d", 2), ("band_3", 0), ("band_9", 0), ("band_9", 1), ("band_31", 0), ("band_31", 2)]
+
+
+@pytest.mark.parametrize("name,grid", CASES)
+@pytest.mark.parametrize("tau", [None, 0.0, 2.0 ** -24, 2.0 ** -11])
+def test_gpu_planes_equal_slabs(gpu, orc, name, grid, tau):
+    """Iterations and x on the planes equal those on the slabs: 5-, 7- and
+    27-point stencils and bands whose tables are padded, sizes that end inside
+    a tile row and a row slot, one to eight rows per thread, one workgroup and
+    several, values of each class."""
+    rp, ci, va = _matrix(gpu, name)
+    n = len(rp) - 1
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, n))
+    A, S = gpu.Matrix(rp, ci, va), gpu.Matrix(rp, ci, va)
+    S.set_index_width(2)
+    prec = dict(precision=gpu.MF_FP64) if tau is None else dict(precision=gpu.MF_MIXED, tau=tau, rr_factor=1e-2)
+    for method in (gpu.MF_CG, gpu.MF_BICGSTAB):
+        if method == gpu.MF_CG and name.startswith("convdiff"):
+            continue
+        o = dict(method=method, tol=TOL, grid=grid, **prec)
+        print(f"case {name} grid={grid} tau={tau} method={method}", flush=True)
+        x, rep = A.solve(b, **o)
+        y, sep = S.solve(b, **o)
+        assert rep["status"] == 0 and rep["relres_true"] <= TOL, rep
+        assert (rep["iterations"], rep["replacements"], rep["grid"]) == (sep["iterations"], sep["replacements"], sep["grid"])
+        assert np.array_equal(x, y)
+        x2, _ = A.solve(b, **o)
+        assert np.array_equal(x, x2)
+
+
+def test_gpu_planes_beyond_register_x(gpu, orc):
+    """17 to 36 rows per thread, where x stays in the caller's buffer (the
+    vectors count as streamed): 3, 4 and 5 workgroups of 8704 to 18432 rows
+    give the solution of the default grid and its iterations within one."""
+    rp, ci, va = gpu.gen_poisson3d(34, 33, 32)
+    n = len(rp) - 1
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(2).uniform(-1, 1, n))
+    A = gpu.Matrix(rp, ci, va)
+    for prec in (dict(precision=gpu.MF_FP64), dict(precision=gpu.MF_MIXED, tau=0.0, rr_factor=1e-4)):
+        y, sep = A.solve(b, tol=TOL, **prec)
+        for grid in (2, 3, 4):
+            print(f"case poisson3d_34x33x32 grid={grid} {prec}", flush=True)
+            x, rep = A.solve(b, tol=TOL, grid=grid, **prec)
+            assert rep["status"] == 0 and rep["relres_true"] <= TOL and rep["streamed"] == 1
+            assert abs(rep["iterations"] - sep["iterations"]) <= max(2, 0.05 * sep["iterations"])
+            assert np.linalg.norm(x - y) <= 1e-8 * np.linalg.norm(y)
