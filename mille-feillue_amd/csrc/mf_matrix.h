@@ -51,6 +51,8 @@ struct Layout {
 struct Workspace {
     size_t ncol = 0;
     int G = 0;
+    uint8_t *block = nullptr;  // the allocation behind g64 .. red
+    int ring = 1;  // copies of the published vector in g64 and g32, ncol entries apart
     double *g64 = nullptr, *h64 = nullptr, *q64 = nullptr;
     float *g32 = nullptr;
     unsigned long long *slots = nullptr;

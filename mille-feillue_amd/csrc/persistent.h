@@ -34,8 +34,13 @@ struct SolveArgs {
     int nrows, crows;  // rows of the system and of a chunk (tilem and trw tile rows)
     const double *b;
     double *x;
-    double *g64;       // published Krylov vector (FP64)
-    float *g32;        // its FP32 copy for low-precision tiles
+    // the published Krylov vector (FP64) and its FP32 copy for low-precision
+    // tiles: ring copies of each, rstride entries apart, written in turn (see
+    // Reducer)
+    double *g64;
+    float *g32;
+    int ring;
+    long long rstride;
     double *h64, *q64; // publishing slots of the true-residual pass
     unsigned long long *slots;  // sync words [SLOT_BUFS][G][SLOT_WORDS]
     int *ctl;          // 0 abort, 1 status, 2 iterations, 3 replacements
@@ -115,12 +120,29 @@ static_assert(SYNC_K <= SLOT_WORDS, "sync line");
 // workgroup waits for its own earlier stores (the emptying among them) to
 // complete, so a reader that has seen a workgroup's epoch e + 1 words finds
 // its epoch e + 2 line either empty or current.
-// publish: vector entries written before the sync (with st_agent) are read
-// by other workgroups after it -- each wave drains its stores before the
-// workgroup barrier that precedes the sync words, and the readers invalidate
-// their caches (agent-scope acquire) after the poll.  The wait is bounded:
-// after spin_limit polls the workgroup raises the abort word and every
-// workgroup leaves (returns false).
+// Flags: SY_DRAIN -- vector entries written before the sync (with st_agent)
+// are read by other workgroups after it: each wave drains its stores before
+// the workgroup barrier that precedes the sync words.  SY_ACQ -- the readers
+// invalidate their caches (agent-scope acquire) after the poll.
+// The published vector rotates through A.ring copies, and only the syncs that
+// publish copy 0 carry SY_ACQ.  A copy's entries are gathered in the product
+// after their sync and not again until the copy is rewritten, ring syncs
+// later; in between lie an allreduce that every workgroup reaches only after
+// that product, and then an invalidation by this workgroup (L1 and the XCD's
+// L2).  So no cache holds older entries when a copy is gathered again,
+// whichever workgroup of the XCD had brought them in.  That takes grid syncs:
+// with neighbour waits every publish carries SY_ACQ, since a workgroup may read
+// (beside the entries it waits for, in the same cache line or under a value 0)
+// entries that their owner has not written yet, which another workgroup of the
+// XCD would then find in the L2.
+// An invalidation takes the XCD's L2 about 53 ns, one after the other for its
+// workgroups (at every publish it added 1.7 us to a 2.2 us sync of 256
+// workgroups), and drops the rows that the XCD's own workgroups have just
+// written through it (83x79x77 Poisson CG, mixed: 9.6 us per iteration with
+// one copy, 8.5 with four).
+// The wait is bounded: after spin_limit polls the workgroup raises the abort
+// word and every workgroup leaves (returns false).
+constexpr int SY_DRAIN = 1, SY_ACQ = 2, SY_PUBLISH = SY_DRAIN | SY_ACQ;
 template <int TPB, int K>
 struct Reducer {
     static_assert(K <= SYNC_K, "reducer width");
@@ -135,7 +157,7 @@ struct Reducer {
         __device__ void operator()() const {}
     };
     template <int N, typename F = Nothing>
-    __device__ bool allreduce(const SolveArgs &A, double (&v)[N], bool publish, F meanwhile = F())
+    __device__ bool allreduce(const SolveArgs &A, double (&v)[N], int flags, F meanwhile = F())
     {
         static_assert(N >= 1 && N <= K, "reducer width");
         const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -144,7 +166,7 @@ struct Reducer {
             double s = wave_sum(v[k]);
             if (lane == 0) s_red[wv * K + k] = s;
         }
-        if (publish) __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
+        if (flags & SY_DRAIN) __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
         __syncthreads();
         ++ep;
         // diagnostic stamps of syncs PHASE_EP0 .. PHASE_EP0 + 3: arrival and
@@ -162,7 +184,7 @@ struct Reducer {
                     for (int w = 0; w < TPB / 64; w++) sum += s_red[w * K + lane];
                     s_bc[lane] = sum;
                 }
-                if (publish) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                if (flags & SY_ACQ) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
             if (stamp) st[1] = wall_clock64();
             __syncthreads();
@@ -236,7 +258,7 @@ struct Reducer {
                     __hip_atomic_store(A.slots + (size_t)((ep + 2) % SLOT_BUFS) * G * SLOT_WORDS +
                                            (size_t)blockIdx.x * SLOT_WORDS + lane,
                                        SLOT_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (publish) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                if (flags & SY_ACQ) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
             if (lane == 0) *s_flag = ab;
         }
@@ -252,18 +274,18 @@ struct Reducer {
     __device__ bool barrier(const SolveArgs &A)
     {
         double z[1] = {0.0};
-        return allreduce(A, z, true);
+        return allreduce(A, z, SY_PUBLISH);
     }
 
     // Publish without a grid rendezvous: after this workgroup's vector stores
     // have drained, its chunk's epoch word is raised, and the workgroup waits
     // only until the chunks its SpMV gathers from show the same epoch (then
-    // invalidates its caches, as after a publishing allreduce).  No vector is
+    // invalidates its caches where the flags ask for it).  No vector is
     // overwritten before the next allreduce, which every workgroup reaches
     // only after its SpMV, so readers never see a later value than the one
     // published here.  Bounded like allreduce.
     unsigned nep = 0;
-    __device__ bool neighbours(const SolveArgs &A, int chunk)
+    __device__ bool neighbours(const SolveArgs &A, int chunk, int flags)
     {
         const int tid = threadIdx.x, lane = tid & 63;
         __builtin_amdgcn_s_waitcnt(0);  // this wave's stores are complete
@@ -290,7 +312,7 @@ struct Reducer {
                 }
                 __builtin_amdgcn_s_sleep(1);
             }
-            if (!ab) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (!ab && (flags & SY_ACQ)) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             if (lane == 0) *s_flag = ab;
         }
         __syncthreads();
@@ -298,9 +320,33 @@ struct Reducer {
     }
 
     // The sync after publishing the vector the next SpMV gathers.
-    __device__ bool published(const SolveArgs &A, int chunk)
+    __device__ bool published(const SolveArgs &A, int chunk, int flags)
     {
-        return A.nbr && A.G > 1 ? neighbours(A, chunk) : barrier(A);
+        double z[1] = {0.0};
+        return A.nbr && A.G > 1 ? neighbours(A, chunk, flags) : allreduce(A, z, flags);
+    }
+};
+
+// The copy of the published vector written last and gathered next.  local:
+// the vector is in this workgroup's LDS, where a barrier publishes it.
+struct RingCursor {
+    double *g64;
+    float *g32;
+    bool local;
+    int slot = 0;
+    __device__ RingCursor(double *g64_, float *g32_, bool local_) : g64(g64_), g32(g32_), local(local_) {}
+    // before the stores of a publish: on to the next copy
+    __device__ void advance(const SolveArgs &A)
+    {
+        if (local) return;
+        slot = slot + 1 < A.ring ? slot + 1 : 0;
+        g64 = A.g64 + slot * A.rstride;
+        g32 = A.g32 + slot * A.rstride;
+    }
+    // flags of the sync that follows those stores
+    __device__ int flags(const SolveArgs &A) const
+    {
+        return local ? 0 : slot == 0 || A.nbr ? SY_PUBLISH : SY_DRAIN;
     }
 };
 
@@ -491,15 +537,16 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
     // the solve, with the gathered vector and the slabs each in LDS or in
     // global memory (up to four inlined copies, each with its address spaces
     // known to the compiler)
-    auto solve = [&](double *g64, float *g32, auto lds_tag, auto slab_tag) {
+    auto solve = [&](double *g64_0, float *g32_0, auto lds_tag, auto slab_tag) {
         constexpr bool lds = decltype(lds_tag)::value, ldsv = decltype(slab_tag)::value;
+        RingCursor ring(g64_0, g32_0, lds);
         auto publish = [&](size_t row, double v) {
             if (lds) {
-                if (A.has64) g64[row] = v;
-                if (A.haslow) g32[row] = (float)v;
+                if (A.has64) ring.g64[row] = v;
+                if (A.haslow) ring.g32[row] = (float)v;
             } else {
-                if (A.has64) st_agent(g64 + row, v);
-                if (A.haslow) st_agent(g32 + row, (float)v);
+                if (A.has64) st_agent(ring.g64 + row, v);
+                if (A.haslow) st_agent(ring.g32 + row, (float)v);
             }
         };
         auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
@@ -533,7 +580,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 v1[0] += bv * bv;
             }
         }
-        if (!R.allreduce(A, v1, true)) return;
+        if (!R.allreduce(A, v1, ring.flags(A))) return;
         const double bnorm2 = v1[0];
         if (blockIdx.x == 0 && tid == 0) A.out[0] = sqrt(bnorm2);
         const double tol2 = A.tol * A.tol * bnorm2;
@@ -558,6 +605,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                     }
                 if (!R.barrier(A)) return;
                 double t1[1] = {0.0};
+                ring.advance(A);
     #pragma unroll 1
                 for (int i = 0; i < RPT; i++)
                     if (live(i)) {
@@ -580,9 +628,9 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 if constexpr (r_regs) {
     #pragma clang loop unroll(full)
                     for (int i = 0; i < RPT; i++)
-                        if (live(i)) r_at(i) = A.g64[row_of(i)];
+                        if (live(i)) r_at(i) = (lds || !A.has64 ? A.g64 : ring.g64)[row_of(i)];
                 }
-                if (!R.allreduce(A, t1, true)) return;
+                if (!R.allreduce(A, t1, ring.flags(A))) return;
                 clk.lap(4);
                 ++repl;
                 if (!isfinite(t1[0])) { finish(MF_E_NONFINITE, iter, repl, t1[0], gamma); return; }
@@ -608,7 +656,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
             // per thread -- at 16 the registers spill; BiCGSTAB's allow four
             // only for FP64)
             op.template product<ldsv, RPT <= 8 ? 4 : 2, RPT <= 8 ? 4 : 1>(
-                A, rbase, g64, g32,
+                A, rbase, ring.g64, ring.g32,
                 [&](int i, double w) { s_s[i * TPB + tid] = w + beta * s_s[i * TPB + tid]; });
             // p = r + beta p; (p, s)
             double red[1] = {0.0};
@@ -619,7 +667,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
             clk.lap(0);
-            if (!R.allreduce(A, red, false)) return;
+            if (!R.allreduce(A, red, 0)) return;
             clk.lap(1);
             const double denom = red[0];
             if (!isfinite(denom)) { finish(MF_E_NONFINITE, iter, repl, -1.0, gamma); return; }
@@ -632,6 +680,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
             }
             const double alpha = gamma / denom;
             double g1[1] = {0.0};
+            ring.advance(A);
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) {
                 if constexpr (!x_hbm) xr[i] = xr[i] + alpha * pr[i];
@@ -653,7 +702,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                     }
                 }
             };
-            if (!R.allreduce(A, g1, true, update_x)) return;
+            if (!R.allreduce(A, g1, ring.flags(A), update_x)) return;
             clk.lap(3);
             gamma = g1[0];
         }
@@ -725,15 +774,16 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
     // the solve, with the gathered vector and the slabs each in LDS or in
     // global memory (up to four inlined copies, each with its address spaces
     // known to the compiler)
-    auto solve = [&](double *g64, float *g32, auto lds_tag, auto slab_tag) {
+    auto solve = [&](double *g64_0, float *g32_0, auto lds_tag, auto slab_tag) {
         constexpr bool lds = decltype(lds_tag)::value, ldsv = decltype(slab_tag)::value;
+        RingCursor ring(g64_0, g32_0, lds);
         auto publish = [&](size_t row, double v) {
             if (lds) {
-                if (A.has64) g64[row] = v;
-                if (A.haslow) g32[row] = (float)v;
+                if (A.has64) ring.g64[row] = v;
+                if (A.haslow) ring.g32[row] = (float)v;
             } else {
-                if (A.has64) st_agent(g64 + row, v);
-                if (A.haslow) st_agent(g32 + row, (float)v);
+                if (A.has64) st_agent(ring.g64 + row, v);
+                if (A.haslow) st_agent(ring.g32 + row, (float)v);
             }
         };
         auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
@@ -749,7 +799,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             }
         };
         auto spmv_into = [&](double *dst) {
-            op.template product<ldsv, 2, 4>(A, rbase, g64, g32, [&](int i, double w) { dst[i * TPB + tid] = w; });
+            op.template product<ldsv, 2, 4>(A, rbase, ring.g64, ring.g32, [&](int i, double w) { dst[i * TPB + tid] = w; });
         };
 
         double v1[1] = {0.0};
@@ -765,7 +815,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
                 v1[0] += rr[i] * rr[i];
             }
         }
-        if (!R.allreduce(A, v1, true)) return;
+        if (!R.allreduce(A, v1, ring.flags(A))) return;
         const double bnorm2 = v1[0];
         if (blockIdx.x == 0 && tid == 0) A.out[0] = sqrt(bnorm2);
         const double tol2 = A.tol * A.tol * bnorm2;
@@ -781,17 +831,18 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             double a1[1] = {0.0};
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) a1[0] += rh[i] * s_v[i * TPB + tid];
-            if (!R.allreduce(A, a1, false)) return;
+            if (!R.allreduce(A, a1, 0)) return;
             clk.lap(1);
             if (!(a1[0] != 0.0) || !isfinite(a1[0])) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, -1.0); return; }
             const double alpha = rho / a1[0];
+            ring.advance(A);
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) {
                 sr[i] = rr[i] - alpha * s_v[i * TPB + tid];
                 if (live(i)) publish(row_of(i), sr[i]);
             }
             clk.lap(2);
-            if (!R.published(A, chunk)) return;
+            if (!R.published(A, chunk, ring.flags(A))) return;
             clk.lap(3);
             spmv_into(s_t);  // t = A s
             clk.lap(0);
@@ -805,7 +856,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
                 a2[3] += rh[i] * t;
                 a2[4] += sr[i] * sr[i];
             }
-            if (!R.allreduce(A, a2, false)) return;
+            if (!R.allreduce(A, a2, 0)) return;
             clk.lap(1);
             const double omega = a2[1] > 0.0 ? a2[0] / a2[1] : 0.0;
     #pragma clang loop unroll(full)
@@ -841,7 +892,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
                         t2[0] += rr[i] * rr[i];
                         t2[1] += rr[i] * rh[i];
                     }
-                if (!R.allreduce(A, t2, false)) return;
+                if (!R.allreduce(A, t2, 0)) return;
                 clk.lap(4);
                 ++repl;
                 if (!isfinite(t2[0])) { finish(MF_E_NONFINITE, iter, repl, t2[0], g2); return; }
@@ -856,6 +907,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             if (omega == 0.0 || rho == 0.0) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, g2); return; }
             const double beta = restart ? 0.0 : (rho_new / rho) * (alpha / omega);
             restart = false;
+            ring.advance(A);
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) {
                 pr[i] = rr[i] + beta * (pr[i] - omega * s_v[i * TPB + tid]);
@@ -863,7 +915,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             }
             rho = rho_new;
             clk.lap(2);
-            if (!R.published(A, chunk)) return;
+            if (!R.published(A, chunk, ring.flags(A))) return;
             clk.lap(3);
         }
     };
@@ -996,9 +1048,10 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
     double *__restrict__ vr = A.vec, *__restrict__ vp = A.vec + A.vstride, *__restrict__ vs = A.vec + 2 * A.vstride;
     double *__restrict__ x = A.x;
     int hw0 = -1;
+    RingCursor ring(A.g64, A.g32, false);
     auto publish = [&](size_t row, double v) {
-        if (A.has64) st_agent(A.g64 + row, v);
-        if (A.haslow) st_agent(A.g32 + row, (float)v);
+        if (A.has64) st_agent(ring.g64 + row, v);
+        if (A.haslow) st_agent(ring.g32 + row, (float)v);
     };
     auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
         if (blockIdx.x == 0 && tid == 0) {
@@ -1019,7 +1072,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
         publish(row, bv);
         v1[0] += bv * bv;
     }
-    if (!R.allreduce(A, v1, true)) return;
+    if (!R.allreduce(A, v1, ring.flags(A))) return;
     const double bnorm2 = v1[0];
     if (blockIdx.x == 0 && tid == 0) A.out[0] = sqrt(bnorm2);
     const double tol2 = A.tol * A.tol * bnorm2;
@@ -1040,6 +1093,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
             }
             if (!R.barrier(A)) return;
             double t1[1] = {0.0};
+            ring.advance(A);
             const double *g[2] = {A.h64, A.q64};
             stream_spmv_f64<B, IW, TPB, 2>(A, tr0, tr1, g, [&](size_t row, const double(&acc)[2]) {
                 const double rv = A.b[row] - acc[0];
@@ -1048,7 +1102,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
                 publish(row, rv);
                 t1[0] += rv * rv;
             });
-            if (!R.allreduce(A, t1, true)) return;
+            if (!R.allreduce(A, t1, ring.flags(A))) return;
             clk.lap(4);
             ++repl;
             if (!isfinite(t1[0])) { finish(MF_E_NONFINITE, iter, repl, t1[0], gamma); return; }
@@ -1068,7 +1122,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
         const double beta = fresh ? 0.0 : gamma / gprev;
         // w = A r; s = w + beta s; p = r + beta p; (p, s)
         double red[1] = {0.0};
-        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, A.g64, A.g32, [&](size_t row, double w) {
+        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, ring.g64, ring.g32, [&](size_t row, double w) {
             const double s = w + beta * vs[row];
             vs[row] = s;
             const double p = vr[row] + beta * vp[row];
@@ -1076,7 +1130,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
             red[0] += p * s;
         });
         clk.lap(0);
-        if (!R.allreduce(A, red, false)) return;
+        if (!R.allreduce(A, red, 0)) return;
         clk.lap(1);
         const double denom = red[0];
         if (!isfinite(denom)) { finish(MF_E_NONFINITE, iter, repl, -1.0, gamma); return; }
@@ -1087,6 +1141,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
         }
         const double alpha = gamma / denom;
         double g1[1] = {0.0};
+        ring.advance(A);
         for (size_t row = row0; row < row1; row += TPB) {
             const double p = vp[row];
             x[row] = x[row] + alpha * p;
@@ -1098,7 +1153,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg_st(SolveArgs A)
         gprev = gamma;
         ++iter;
         clk.lap(2);
-        if (!R.allreduce(A, g1, true)) return;
+        if (!R.allreduce(A, g1, ring.flags(A))) return;
         clk.lap(3);
         gamma = g1[0];
     }
@@ -1125,9 +1180,10 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
     double *__restrict__ vs = A.vec + 3 * S, *__restrict__ vv = A.vec + 4 * S, *__restrict__ vt = A.vec + 5 * S;
     double *__restrict__ x = A.x;
     int hw0 = -1;
+    RingCursor ring(A.g64, A.g32, false);
     auto publish = [&](size_t row, double v) {
-        if (A.has64) st_agent(A.g64 + row, v);
-        if (A.haslow) st_agent(A.g32 + row, (float)v);
+        if (A.has64) st_agent(ring.g64 + row, v);
+        if (A.haslow) st_agent(ring.g32 + row, (float)v);
     };
     auto finish = [&](int status, int iter, int repl, double rt2, double g2) {
         if (blockIdx.x == 0 && tid == 0) {
@@ -1147,7 +1203,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
         publish(row, bv);
         v1[0] += bv * bv;
     }
-    if (!R.allreduce(A, v1, true)) return;
+    if (!R.allreduce(A, v1, ring.flags(A))) return;
     const double bnorm2 = v1[0];
     if (blockIdx.x == 0 && tid == 0) A.out[0] = sqrt(bnorm2);
     const double tol2 = A.tol * A.tol * bnorm2;
@@ -1159,26 +1215,27 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
     for (;;) {
         // v = A p; (r^, v)
         double a1[1] = {0.0};
-        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, A.g64, A.g32, [&](size_t row, double w) {
+        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, ring.g64, ring.g32, [&](size_t row, double w) {
             vv[row] = w;
             a1[0] += vrh[row] * w;
         });
         clk.lap(0);
-        if (!R.allreduce(A, a1, false)) return;
+        if (!R.allreduce(A, a1, 0)) return;
         clk.lap(1);
         if (!(a1[0] != 0.0) || !isfinite(a1[0])) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, -1.0); return; }
         const double alpha = rho / a1[0];
+        ring.advance(A);
         for (size_t row = row0; row < row1; row += TPB) {
             const double s = vr[row] - alpha * vv[row];
             vs[row] = s;
             publish(row, s);
         }
         clk.lap(2);
-        if (!R.published(A, chunk)) return;
+        if (!R.published(A, chunk, ring.flags(A))) return;
         clk.lap(3);
         // t = A s; (t, s), (t, t), (r^, s), (r^, t), (s, s)
         double a2[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, A.g64, A.g32, [&](size_t row, double t) {
+        stream_spmv<B, IW, TPB>(A, s_h, s_t0, hw0, tr0, tr1, ring.g64, ring.g32, [&](size_t row, double t) {
             vt[row] = t;
             const double s = vs[row], rh = vrh[row];
             a2[0] += t * s;
@@ -1188,7 +1245,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
             a2[4] += s * s;
         });
         clk.lap(0);
-        if (!R.allreduce(A, a2, false)) return;
+        if (!R.allreduce(A, a2, 0)) return;
         clk.lap(1);
         const double omega = a2[1] > 0.0 ? a2[0] / a2[1] : 0.0;
         for (size_t row = row0; row < row1; row += TPB) {
@@ -1213,7 +1270,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
                 t2[0] += r * r;
                 t2[1] += r * vrh[row];
             });
-            if (!R.allreduce(A, t2, false)) return;
+            if (!R.allreduce(A, t2, 0)) return;
             clk.lap(4);
             ++repl;
             if (!isfinite(t2[0])) { finish(MF_E_NONFINITE, iter, repl, t2[0], g2); return; }
@@ -1228,6 +1285,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
         if (omega == 0.0 || rho == 0.0) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, g2); return; }
         const double beta = restart ? 0.0 : (rho_new / rho) * (alpha / omega);
         restart = false;
+        ring.advance(A);
         for (size_t row = row0; row < row1; row += TPB) {
             const double p = vr[row] + beta * (vp[row] - omega * vv[row]);
             vp[row] = p;
@@ -1235,7 +1293,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab_st(SolveArgs A)
         }
         rho = rho_new;
         clk.lap(2);
-        if (!R.published(A, chunk)) return;
+        if (!R.published(A, chunk, ring.flags(A))) return;
         clk.lap(3);
     }
 }

@@ -160,36 +160,54 @@ static KernelChoice pick(int B, int iw, int method, long long rows_per_wg, bool 
 
 void Workspace::release()
 {
-    void *ps[] = {g64, h64, q64, g32, slots, ctl, out, r_outer, d, tmp, red, dep_ptr, dep_idx, flags, vec};
+    void *ps[] = {block, dep_ptr, dep_idx, flags, vec};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     *this = Workspace();
 }
 
+// Copies of the published vector: 1, 2, 4 and 8 measured (us per iteration,
+// 83x79x77 and 128^3 Poisson CG mixed, 251x257 Laplacian CG FP64): 9.63 / 9.05 /
+// 8.50 / 8.31, 13.5 / 13.0 / 12.7 / 12.7, 7.04 / 6.74 / 6.58 / 6.50.
+constexpr int RING = 4;
+
+// One allocation for all buffers of the matrix's solves (a solve of a new
+// matrix pays for it).
 static int ensure_ws(mf_matrix m, int G)
 {
     Workspace &w = m->ws;
     const size_t ncol = (size_t)std::max(m->tilem, m->tilen) * m->B;
-    if (w.ncol >= ncol && w.G >= G && w.g64) return MF_OK;
+    if (w.ncol >= ncol && w.G >= G && w.block) return MF_OK;
     w.release();
     w.ncol = ncol;
     w.G = std::max(G, 1);
-    MF_HIP(hipMalloc((void **)&w.g64, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.h64, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.q64, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.g32, sizeof(float) * ncol));
-    MF_HIP(hipMalloc((void **)&w.slots, sizeof(unsigned long long) * SLOT_BUFS * SLOT_WORDS * w.G));
-    MF_HIP(hipMalloc((void **)&w.ctl, sizeof(int) * 8));
-    MF_HIP(hipMalloc((void **)&w.out, sizeof(double) * 4));
-    MF_HIP(hipMalloc((void **)&w.r_outer, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.d, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.tmp, sizeof(double) * ncol));
-    MF_HIP(hipMalloc((void **)&w.red, sizeof(double) * (ncol / 16 + 1024)));
+    w.ring = RING;
+    size_t size = 0;
+    auto take = [&](size_t bytes) {
+        const size_t at = size;
+        size += (bytes + 255) / 256 * 256;
+        return at;
+    };
+    // the gathered vectors first: cleared below
+    const size_t g64 = take(sizeof(double) * ncol * w.ring), h64 = take(sizeof(double) * ncol),
+                 q64 = take(sizeof(double) * ncol), g32 = take(sizeof(float) * ncol * w.ring), gathered = size,
+                 slots = take(sizeof(unsigned long long) * SLOT_BUFS * SLOT_WORDS * w.G), ctl = take(sizeof(int) * 8),
+                 out = take(sizeof(double) * 4), r_outer = take(sizeof(double) * ncol), d = take(sizeof(double) * ncol),
+                 tmp = take(sizeof(double) * ncol), red = take(sizeof(double) * (ncol / 16 + 1024));
+    MF_HIP(hipMalloc((void **)&w.block, size));
+    w.g64 = reinterpret_cast<double *>(w.block + g64);
+    w.h64 = reinterpret_cast<double *>(w.block + h64);
+    w.q64 = reinterpret_cast<double *>(w.block + q64);
+    w.g32 = reinterpret_cast<float *>(w.block + g32);
+    w.slots = reinterpret_cast<unsigned long long *>(w.block + slots);
+    w.ctl = reinterpret_cast<int *>(w.block + ctl);
+    w.out = reinterpret_cast<double *>(w.block + out);
+    w.r_outer = reinterpret_cast<double *>(w.block + r_outer);
+    w.d = reinterpret_cast<double *>(w.block + d);
+    w.tmp = reinterpret_cast<double *>(w.block + tmp);
+    w.red = reinterpret_cast<double *>(w.block + red);
     // gather vectors are read up to tilen*B; entries beyond the rows stay zero
-    MF_HIP(hipMemset(w.g64, 0, sizeof(double) * ncol));
-    MF_HIP(hipMemset(w.g32, 0, sizeof(float) * ncol));
-    MF_HIP(hipMemset(w.h64, 0, sizeof(double) * ncol));
-    MF_HIP(hipMemset(w.q64, 0, sizeof(double) * ncol));
+    MF_HIP(hipMemset(w.block, 0, gathered));
     return MF_OK;
 }
 
@@ -325,6 +343,8 @@ struct WsView {
     const int *dep_ptr = nullptr, *dep_idx = nullptr;
     unsigned *flags = nullptr;
     int dep_max = -1;
+    int ring = 1;  // copies of the published vector, rstride entries apart
+    long long rstride = 0;
     double *vec = nullptr;
     long long vstride = 0;
     bool allow_profile = true;  // the phase clock allocates its buffer on first use
@@ -369,6 +389,8 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     A.x = d_x;
     A.g64 = w.g64;
     A.g32 = w.g32;
+    A.ring = w.ring;
+    A.rstride = w.rstride;
     A.h64 = w.h64;
     A.q64 = w.q64;
     A.slots = w.slots;
@@ -529,6 +551,8 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
         w.flags = ws.flags;
         w.dep_max = ws.dep_max;
     }
+    w.ring = ws.ring;
+    w.rstride = (long long)ws.ncol;
     w.vec = ws.vec;
     w.vstride = (long long)ws.ncol;
     return launch_persistent(m, L, L64, method, d_b, d_x, tol, o, G, trw, kc, w, sync, res, grid_out, block_out,
