@@ -496,6 +496,8 @@ template <int B, int IW, int CM = CM_ALL> struct Slabs {
 // rather than recurred (Chronopoulos-Gear's (A r, r) - beta (r, r) / alpha
 // form), which holds after a residual replacement that keeps the direction
 // and, with lossy tiles, halves the iterations on rough coefficients.
+// The sums over a thread's rows are explicit fused chains: left to contraction,
+// the first two squares of an unrolled chain may fuse either way.
 template <class M, int TPB, int RPT>
 __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
 {
@@ -577,7 +579,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 r_at(i) = bv;
                 if constexpr (x_hbm) A.x[row] = 0.0;
                 publish(row, bv);
-                v1[0] += bv * bv;
+                v1[0] = fma_t(bv, bv, v1[0]);
             }
         }
         if (!R.allreduce(A, v1, ring.flags(A))) return;
@@ -623,7 +625,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                         } else {
                             r_at(i) = rv;
                         }
-                        t1[0] += rv * rv;
+                        t1[0] = fma_t(rv, rv, t1[0]);
                     }
                 if constexpr (r_regs) {
     #pragma clang loop unroll(full)
@@ -663,7 +665,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) {
                 pr[i] = r_at(i) + beta * pr[i];
-                red[0] += pr[i] * s_s[i * TPB + tid];
+                red[0] = fma_t(pr[i], s_s[i * TPB + tid], red[0]);
                 if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
             clk.lap(0);
@@ -687,7 +689,7 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                 const double rv = r_at(i) - alpha * s_s[i * TPB + tid];
                 r_at(i) = rv;
                 if (live(i)) publish(row_of(i), rv);
-                g1[0] += rv * rv;
+                g1[0] = fma_t(rv, rv, g1[0]);
                 if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
             gprev = gamma;
@@ -812,7 +814,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
                 const size_t row = row_of(i);
                 rr[i] = rh[i] = pr[i] = A.b[row];
                 publish(row, pr[i]);
-                v1[0] += rr[i] * rr[i];
+                v1[0] = fma_t(rr[i], rr[i], v1[0]);
             }
         }
         if (!R.allreduce(A, v1, ring.flags(A))) return;
@@ -830,7 +832,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
             clk.lap(0);
             double a1[1] = {0.0};
     #pragma clang loop unroll(full)
-            for (int i = 0; i < RPT; i++) a1[0] += rh[i] * s_v[i * TPB + tid];
+            for (int i = 0; i < RPT; i++) a1[0] = fma_t(rh[i], s_v[i * TPB + tid], a1[0]);
             if (!R.allreduce(A, a1, 0)) return;
             clk.lap(1);
             if (!(a1[0] != 0.0) || !isfinite(a1[0])) { finish(MF_E_BREAKDOWN, iter, repl, -1.0, -1.0); return; }
@@ -850,11 +852,11 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
     #pragma clang loop unroll(full)
             for (int i = 0; i < RPT; i++) {
                 const double t = s_t[i * TPB + tid];
-                a2[0] += t * sr[i];
-                a2[1] += t * t;
-                a2[2] += rh[i] * sr[i];
-                a2[3] += rh[i] * t;
-                a2[4] += sr[i] * sr[i];
+                a2[0] = fma_t(t, sr[i], a2[0]);
+                a2[1] = fma_t(t, t, a2[1]);
+                a2[2] = fma_t(rh[i], sr[i], a2[2]);
+                a2[3] = fma_t(rh[i], t, a2[3]);
+                a2[4] = fma_t(sr[i], sr[i], a2[4]);
             }
             if (!R.allreduce(A, a2, 0)) return;
             clk.lap(1);
@@ -889,8 +891,8 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
                 for (int i = 0; i < RPT; i++)
                     if (live(i)) {
                         rr[i] = s_t[i * TPB + tid];
-                        t2[0] += rr[i] * rr[i];
-                        t2[1] += rr[i] * rh[i];
+                        t2[0] = fma_t(rr[i], rr[i], t2[0]);
+                        t2[1] = fma_t(rr[i], rh[i], t2[1]);
                     }
                 if (!R.allreduce(A, t2, 0)) return;
                 clk.lap(4);
