@@ -1144,7 +1144,7 @@ static int batch_assign(mf_batch_s *bt, int g_target, const std::vector<int> &it
     bt->d_wg = nullptr;
     bt->d_slots = nullptr;
     MF_HIP(hipMalloc((void **)&bt->d_wg, sizeof(int) * h.size()));
-    MF_HIP(hipMemcpy(bt->d_wg, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice));
+    MF_HIP(upload(bt->d_wg, h.data(), sizeof(int) * h.size()));
     MF_HIP(hipMalloc((void **)&bt->d_slots, sizeof(unsigned long long) * 2 * 2 * BK_MAXV * (size_t)G));
     bt->G = G;
     bt->nlines = G;
@@ -1209,7 +1209,7 @@ static int batch_assign_oc(mf_batch_s *bt, const std::vector<int> &iters)
     bt->d_wg = nullptr;
     bt->d_slots = nullptr;
     MF_HIP(hipMalloc((void **)&bt->d_wg, sizeof(int) * h.size()));
-    MF_HIP(hipMemcpy(bt->d_wg, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice));
+    MF_HIP(upload(bt->d_wg, h.data(), sizeof(int) * h.size()));
     MF_HIP(hipMalloc((void **)&bt->d_slots, sizeof(unsigned long long) * 2 * 2 * BK_MAXV * (size_t)line));
     bt->G = G;
     bt->nlines = line;
@@ -1254,7 +1254,7 @@ static int batch_capture(mf_batch_s *bt)
         if (bt->d_prof) (void)hipFree(bt->d_prof);
         bt->d_prof = nullptr;
         MF_HIP(hipMalloc((void **)&bt->d_prof, sizeof(unsigned long long) * 4 * bt->G));
-        MF_HIP(hipMemset(bt->d_prof, 0, sizeof(unsigned long long) * 4 * bt->G));
+        MF_HIP(hipMemsetAsync(bt->d_prof, 0, sizeof(unsigned long long) * 4 * bt->G, st));
         A.prof = bt->d_prof;
     }
     bt->fn = bt->oc ? pick_batched_oc(bt->B, bt->iw) : pick_batched(bt->B, bt->iw, bt->K);
@@ -1365,8 +1365,8 @@ static int batch_build(mf_batch_s *bt)
     const size_t vn = bt->rows * bt->K;
     MF_HIP(hipMalloc((void **)&bt->d_vec, sizeof(double) * 5 * vn));
     MF_HIP(hipMalloc((void **)&bt->d_r32, sizeof(float) * vn));
-    MF_HIP(hipMemset(bt->d_vec, 0, sizeof(double) * 5 * vn));
-    MF_HIP(hipMemset(bt->d_r32, 0, sizeof(float) * vn));
+    MF_HIP(hipMemsetAsync(bt->d_vec, 0, sizeof(double) * 5 * vn, st));
+    MF_HIP(hipMemsetAsync(bt->d_r32, 0, sizeof(float) * vn, st));
     MF_HIP(hipMalloc((void **)&bt->d_ctl, sizeof(int) * 8));
     MF_HIP(hipMalloc((void **)&bt->d_sys_out, sizeof(int) * 4 * bt->nsys));
     MF_HIP(hipMalloc((void **)&bt->d_relres, sizeof(double) * bt->nsys));
@@ -1631,7 +1631,7 @@ int mf_batch_solve(mf_batch bt, const double *const *b, double *const *x, int *i
                 std::fprintf(stderr, "\n");
             }
         }
-        MF_HIP(hipMemset(bt->args.prof, 0, sizeof(unsigned long long) * pf.size()));
+        MF_HIP(hipMemsetAsync(bt->args.prof, 0, sizeof(unsigned long long) * pf.size(), stream()));
     }
     return oc.status == MF_E_TIMEOUT ? fail(MF_E_TIMEOUT, "group sync timeout") : MF_OK;
 }

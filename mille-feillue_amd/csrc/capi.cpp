@@ -186,13 +186,13 @@ int mf_matrix_create(int rowA, int colA, int nnz, const int *rowptr, const int *
         hipMalloc((void **)&m->d_col, sizeof(int) * nzs) != hipSuccess ||
         hipMalloc((void **)&m->d_val, sizeof(double) * nzs) != hipSuccess)
         return bail(fail(MF_E_NOMEM, "device allocation of the CSR"));
-    if (hipMemcpy(m->d_rowptr, rowptr, sizeof(int) * (rowA + 1), hipMemcpyHostToDevice) != hipSuccess ||
-        (nz && hipMemcpy(m->d_col, colidx, sizeof(int) * nz, hipMemcpyHostToDevice) != hipSuccess) ||
-        (nz && hipMemcpy(m->d_val, val, sizeof(double) * nz, hipMemcpyHostToDevice) != hipSuccess))
+    if (upload(m->d_rowptr, rowptr, sizeof(int) * (rowA + 1)) != hipSuccess ||
+        upload(m->d_col, colidx, sizeof(int) * (size_t)nz) != hipSuccess ||
+        upload(m->d_val, val, sizeof(double) * (size_t)nz) != hipSuccess)
         return bail(fail(MF_E_HIP, "upload of the CSR"));
     if (val_low) {
         if (hipMalloc((void **)&m->d_val_low, sizeof(float) * nzs) != hipSuccess ||
-            (nz && hipMemcpy(m->d_val_low, val_low, sizeof(float) * nz, hipMemcpyHostToDevice) != hipSuccess))
+            upload(m->d_val_low, val_low, sizeof(float) * (size_t)nz) != hipSuccess)
             return bail(fail(MF_E_HIP, "upload of the low values"));
     }
     rc = build_reference_tiles(m);
@@ -400,8 +400,8 @@ int mf_spmv(mf_matrix m, int mixed, const double *x, double *y)
     double *dx = nullptr, *dy = nullptr;
     MF_HIP(hipMalloc((void **)&dx, sizeof(double) * nc));
     MF_HIP(hipMalloc((void **)&dy, sizeof(double) * nr));
-    MF_HIP(hipMemset(dx, 0, sizeof(double) * nc));
-    MF_HIP(hipMemcpy(dx, x, sizeof(double) * m->colA, hipMemcpyHostToDevice));
+    MF_HIP(hipMemsetAsync(dx, 0, sizeof(double) * nc, stream()));
+    MF_HIP(upload(dx, x, sizeof(double) * m->colA));
     int rc = spmv_device(m, L, dx, dy, true);
     if (!rc) {
         if (hipStreamSynchronize(stream()) != hipSuccess ||
@@ -428,7 +428,7 @@ int mf_spmv_bench(mf_matrix m, int mixed, int reps, double *ms)
     MF_HIP(hipMalloc((void **)&dx, sizeof(double) * nc));
     MF_HIP(hipMalloc((void **)&dy, sizeof(double) * nr));
     std::vector<double> ones(nc, 1.0);
-    MF_HIP(hipMemcpy(dx, ones.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
+    MF_HIP(upload(dx, ones.data(), sizeof(double) * nc));
     int rc = spmv_device(m, L, dx, dy, true);  // also fills the FP32 copy
     if (rc) return rc;
     hipStream_t st = stream();
@@ -481,7 +481,7 @@ int mf_vendor_solve(mf_matrix m, const double *b, double *x, const mf_opts *o, m
     double *db = nullptr, *dx = nullptr;
     MF_HIP(hipMalloc((void **)&db, sizeof(double) * n));
     MF_HIP(hipMalloc((void **)&dx, sizeof(double) * n));
-    MF_HIP(hipMemcpy(db, b, sizeof(double) * n, hipMemcpyHostToDevice));
+    MF_HIP(upload(db, b, sizeof(double) * n));
     int rc = mf::vendor_solve_device(m, db, dx, *o, rep);
     if (hipMemcpy(x, dx, sizeof(double) * n, hipMemcpyDeviceToHost) != hipSuccess && !rc)
         rc = fail(MF_E_HIP, "copy x");
@@ -499,9 +499,9 @@ int mf_solve(mf_matrix m, const double *b, double *x, const mf_opts *o, mf_repor
     double *db = nullptr, *dx = nullptr;
     MF_HIP(hipMalloc((void **)&db, sizeof(double) * n));
     MF_HIP(hipMalloc((void **)&dx, sizeof(double) * n));
-    MF_HIP(hipMemset(db, 0, sizeof(double) * n));
-    MF_HIP(hipMemset(dx, 0, sizeof(double) * n));
-    MF_HIP(hipMemcpy(db, b, sizeof(double) * m->rowA, hipMemcpyHostToDevice));
+    MF_HIP(hipMemsetAsync(db, 0, sizeof(double) * n, stream()));
+    MF_HIP(hipMemsetAsync(dx, 0, sizeof(double) * n, stream()));
+    MF_HIP(upload(db, b, sizeof(double) * m->rowA));
     int rc = solve_device(m, db, dx, *o, rep);
     if (hipMemcpy(x, dx, sizeof(double) * m->rowA, hipMemcpyDeviceToHost) != hipSuccess && !rc)
         rc = fail(MF_E_HIP, "copy x");

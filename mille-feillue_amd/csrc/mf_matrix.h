@@ -135,6 +135,16 @@ int vendor_solve_device(mf_matrix m, const double *d_b, double *d_x, const mf_op
 int encode_cols_device(mf_matrix m, uint8_t *d_out);  // tiles.hip
 int classes_device(mf_matrix m, double tau, int allow_mask, uint8_t *d_codes);  // tiles.hip
 hipStream_t stream();
+// Host to device on the library's stream, complete on return.  The stream does
+// not synchronise with the null stream, so a plain hipMemcpy or hipMemset
+// (which need not have reached the device when they return: small pageable
+// copies and fills are asynchronous) is not ordered before its kernels.
+inline hipError_t upload(void *dst, const void *src, size_t bytes)
+{
+    if (!bytes) return hipSuccess;
+    const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream());
+    return e != hipSuccess ? e : hipStreamSynchronize(stream());
+}
 // Live handles, so that mf_finalize can release what callers still hold and
 // later destroy calls on released handles do nothing (capi.cpp).
 void live_add(void *h, int kind);     // kind 0 matrix, 1 batch

@@ -207,7 +207,7 @@ static int ensure_ws(mf_matrix m, int G)
     w.tmp = reinterpret_cast<double *>(w.block + tmp);
     w.red = reinterpret_cast<double *>(w.block + red);
     // gather vectors are read up to tilen*B; entries beyond the rows stay zero
-    MF_HIP(hipMemset(w.block, 0, gathered));
+    MF_HIP(hipMemsetAsync(w.block, 0, gathered, stream()));
     return MF_OK;
 }
 

@@ -733,10 +733,10 @@ static int build_reference_tiles_B(mf_matrix m)
             while (P < b - a) P <<= 1;
             off[i + 1] = off[i] + P;
         }
-        MF_HIP(hipMemcpy(big_list, bl.data(), sizeof(int) * nbig, hipMemcpyHostToDevice));
+        MF_HIP(upload(big_list, bl.data(), sizeof(int) * nbig));
         MF_HIP(hipMalloc((void **)&gkeys, sizeof(unsigned long long) * off[nbig]));
         MF_HIP(hipMalloc((void **)&koff, sizeof(long long) * (nbig + 1)));
-        MF_HIP(hipMemcpy(koff, off.data(), sizeof(long long) * (nbig + 1), hipMemcpyHostToDevice));
+        MF_HIP(upload(koff, off.data(), sizeof(long long) * (nbig + 1)));
         k_sort_big<B><<<nbig, 1024, 0, st>>>(m->d_rowptr, m->d_col, m->rowA, big_list, koff, gkeys,
                                             perm, tcount);
         MF_HIP(hipGetLastError());

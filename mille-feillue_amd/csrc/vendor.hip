@@ -133,9 +133,9 @@ static int vendor_setup(mf_matrix m)
     MF_HIP(hipMalloc((void **)&V->rp, sizeof(int) * (n + 1)));
     MF_HIP(hipMalloc((void **)&V->ci, sizeof(int) * ci.size()));
     MF_HIP(hipMalloc((void **)&V->va, sizeof(double) * va.size()));
-    MF_HIP(hipMemcpy(V->rp, rp.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
-    MF_HIP(hipMemcpy(V->ci, ci.data(), sizeof(int) * ci.size(), hipMemcpyHostToDevice));
-    MF_HIP(hipMemcpy(V->va, va.data(), sizeof(double) * va.size(), hipMemcpyHostToDevice));
+    MF_HIP(upload(V->rp, rp.data(), sizeof(int) * (n + 1)));
+    MF_HIP(upload(V->ci, ci.data(), sizeof(int) * ci.size()));
+    MF_HIP(upload(V->va, va.data(), sizeof(double) * va.size()));
     double **vecs[] = {&V->r, &V->p, &V->q, &V->s, &V->t, &V->rh, &V->x};
     for (double **v : vecs) MF_HIP(hipMalloc((void **)v, vb));
     MF_HIP(hipMalloc((void **)&V->sc, sizeof(double) * 16));
