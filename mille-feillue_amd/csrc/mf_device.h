@@ -304,7 +304,10 @@ __device__ __forceinline__ void slab_spmv_rows(const DevL &L, const int4 *hd, co
             for (int k = 0; k < NB; k++) {
                 const int t0 = 0;
                 // index base: the lane's row for a pattern slab, else the tile row's
-                const int tcb = IW != 1 && slab_pattern(h[k].x)
+                // (row 0 without a slab: a tile row past the last one, whose
+                // own rows lie beyond the vector)
+                const int tcb = h[k].y == 0 ? 0
+                                : IW != 1 && slab_pattern(h[k].x)
                                     ? (IW == 2 ? tcr[kb + k] + r : row0 + (kb + k) * QS * B)
                                     : tcr[kb + k];
 #pragma unroll
