@@ -302,21 +302,24 @@ static int ensure_deps(mf_matrix m, int G, int trw)
     return MF_OK;
 }
 
-// One persistent launch: solves L x = b (x overwritten) on the stream.
 // Grid of the persistent solvers: workgroups and tile rows per workgroup.
-// grid > 0 is taken as given; by default one workgroup per CU, but no more
-// than leave every lane group (B lanes of a 512-thread workgroup) two tile
-// rows, since every grid sync polls all workgroups -- except that a system
-// the rule puts on 2 .. CUs/2 - 1 workgroups gets one tile row per lane group
-// on up to half the CUs.
+// grid > 0 is taken as given.  By default a system of up to four tile rows per
+// lane group (B lanes of a 512-thread workgroup) gets one workgroup, which
+// needs no grid syncs.  Others get one tile row per lane group where that takes
+// at most 0.7 of the CUs, else two (every sync polls all workgroups, and the
+// last one of 256 arrives later than that of 128), on at most one workgroup per
+// CU.  Workgroups are filled whole: a chunk that exceeds a multiple of the lane
+// groups by a few tile rows doubles everybody's row slots.  Measured, ms, the
+// rule's workgroups against others: 39^3 27-point BiCGSTAB FP64 116: 1.93 (113:
+// 2.66, 58: 2.51, 232: 2.16), 45^3 178: 2.46 (127: 3.07, 248: 2.61); Poisson CG
+// FP64 33x31x29 58: 1.16 (57: 1.26, 29: 1.25, 116: 1.17), 45^3 178: 1.45 (127:
+// 1.50, 248: 1.56), 55^3 163: 1.86 (160: 2.05, 254: 2.04), 83x79x77 247: 3.43
+// (255: 3.42, 128: 4.24); 251 x 257 Laplacian 126: 5.94 (64: 6.32, 252: 6.76).
 static void solver_grid(int tilem, int B, int grid, int *G_out, int *trw_out)
 {
-    const int cus = device_cu_count();
-    int G = grid > 0 ? grid : std::min(cus, std::max(1, tilem / (2 * (512 / B))));
-    // small systems that still span several workgroups: one tile row per
-    // lane group on up to half the CUs (256^2 Laplacian: 3.8 ms on 128
-    // workgroups against 4.1 on 64 and 5.0 on 256); one workgroup stays one
-    if (grid <= 0 && G > 1 && G < cus / 2) G = std::min(cus / 2, tilem / (512 / B));
+    const int cus = device_cu_count(), per = 512 / B;
+    const int one = (tilem + per - 1) / per, two = (tilem + 2 * per - 1) / (2 * per);
+    int G = grid > 0 ? grid : tilem < 4 * per ? 1 : one <= cus * 7 / 10 ? one : std::min(cus, two);
     G = std::max(1, std::min(G, tilem));
     const int trw = (tilem + G - 1) / G;
     *G_out = (tilem + trw - 1) / trw;  // no empty workgroups
