@@ -10,6 +10,7 @@
 namespace mf {
 
 struct StencilTable;  // stencil.h
+struct PlaneExc;
 int hip_fail(hipError_t e, const char *what);
 #define MF_HIP(call)                                         \
     do {                                                     \
@@ -42,6 +43,8 @@ struct Layout {
     // (ensure_planes; stencil.h)
     uint8_t *planes = nullptr;
     int planes_cls = -1;
+    PlaneExc *exc = nullptr;  // entries of narrower classes, by row
+    int nexc = 0;
     bool planes_tried = false;
     DevL view(const int *tile_ptr) const { return DevL{tile_ptr, trh, stc, blob, split}; }
     void release();

@@ -29,7 +29,9 @@ struct SolveArgs {
     DevL L64;          // FP64 layout for the true-residual passes of a lossy layout
     int use64;         // 1: passes use L64 (headers read from L64) or pl64, else L or pl
     Planes pl, pl64;   // stencil kernels: the layout's planes, and the FP64 ones (use64)
-    const int *off;    // and the offset table
+    const int *off;    // the offset table
+    const PlaneExc *exc;  // the layout's entries outside its planes' class
+    int nexc;
     int tilem, G, trw;
     int nrows, crows;  // rows of the system and of a chunk (tilem and trw tile rows)
     const double *b;
@@ -470,6 +472,7 @@ template <int B, int IW, int CM = CM_ALL> struct Slabs {
                     if (tr0 + (i0 + k) * GPB + grp < tr1) body(i0 + k, w[k]);
             }
         }
+        __device__ void add_listed(double *, const double *, const float *) const {}
         // FP64-accumulated product of row slot i (the true-residual passes)
         template <bool LDSV, int NV>
         __device__ __forceinline__ void pass_row(const SolveArgs &A, int i, size_t, const double *const (&g)[NV],
@@ -802,6 +805,7 @@ __global__ __launch_bounds__(TPB, 1) void k_bicgstab(SolveArgs A)
         };
         auto spmv_into = [&](double *dst) {
             op.template product<ldsv, 2, 4>(A, rbase, ring.g64, ring.g32, [&](int i, double w) { dst[i * TPB + tid] = w; });
+            op.add_listed(dst, ring.g64, ring.g32);
         };
 
         double v1[1] = {0.0};

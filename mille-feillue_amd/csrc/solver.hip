@@ -127,6 +127,7 @@ static int layout_cm(const Layout &L)
 static KernelChoice pick_stencil(mf_matrix m, const Layout &L, const Layout *L64, int method, long long rows_per_wg, int G)
 {
     if (!L.planes || (L64 && L64 != &L && !L64->planes)) return KernelChoice{};
+    if (L.nexc && method == MF_CG) return KernelChoice{};  // see add_listed
     KernelChoice k;
     switch (L.planes_cls) {
     case 0: k = pick_stencil_f64(m->st_L, method, rows_per_wg, G); break;
@@ -379,9 +380,13 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
         A.pl = view(L);
         A.pl64 = A.use64 ? view(*L64) : A.pl;
         A.off = m->d_st->off;
+        A.exc = L.exc;
+        A.nexc = L.nexc;
     } else {
         A.pl = A.pl64 = Planes{};
         A.off = nullptr;
+        A.exc = nullptr;
+        A.nexc = 0;
     }
     A.tilem = m->tilem;
     A.G = G;

@@ -20,7 +20,10 @@
 // 39^3 27-point BiCGSTAB FP64 23.1 -> 21.2; 30 x 31 Laplacian, one workgroup,
 // 3.24 -> 2.97.
 //
-// A plane set holds one class c (0 FP64, 1 FP32, 2 FP16, 3 E4M3), with rows
+// A plane set holds one class c (0 FP64, 1 FP32, 2 FP16, 3 E4M3; layouts of
+// rounded tiles have a few tiles of one or two entries that a narrower class
+// happens to hold: those entries stand in a short list, PlaneExc, sorted by
+// row, and follow the planes' entries of their row, as the slabs sum them), with rows
 // of exactly SW = 5 or 7 entries (5- and 7-point stencils) or, SW = 0, of quads
 // of 4 (any table of up to STENCIL_MAX offsets, padded to a multiple of 4):
 //   FP64  pairs of entries (16 B a row) one after the other, then, when the
@@ -51,6 +54,15 @@ struct StencilTable {
 // with scalar loads (constant address space).
 using OffPtr = const __attribute__((address_space(4))) int *;
 __device__ __forceinline__ OffPtr off_ptr(const int *p) { return (OffPtr)(uintptr_t)p; }
+
+// An entry of a plane set's matrix that another class than the planes' stores
+// (its position there holds 0): value as that class rounds it.
+struct PlaneExc {
+    int row, off;
+    float val;
+    int cls;
+};
+constexpr int EXC_LDS = 64;  // of a chunk, kept in LDS
 
 // Specialised row width of a table of L offsets (0: quads).
 __host__ __device__ constexpr int plane_sw(int L) { return L == 5 || L == 7 ? L : 0; }

@@ -19,7 +19,8 @@ template <int CLS, int SW, bool A64> struct Stencil {
         static constexpr int NE = SW ? SW : 4;
         // LDS left for values beside the vectors, the gathered-vector copy of
         // one-workgroup solves and the reduction scratch
-        static constexpr int VB = (LDS_BYTES - VECS * RPT * TPB * 8 - (RPT <= 4 ? 12 * 2048 : 0) - 1024) / 16 * 16;
+        static constexpr int VB = (LDS_BYTES - VECS * RPT * TPB * 8 - (RPT <= 4 ? 12 * 2048 : 0) - 1024 -
+                                  EXC_LDS * (int)sizeof(PlaneExc)) / 16 * 16;
         // rows (or quads) in flight: what the registers beside the vectors
         // hold, at most 60 loads (the load counter holds 63) and 4 rows
         // (two, three and four rows measure within 3 %, eight 5 % slower)
@@ -31,11 +32,13 @@ template <int CLS, int SW, bool A64> struct Stencil {
         static constexpr int D = FIT < 1 ? 1 : FIT < DMAX ? FIT : DMAX;
         struct Shared {
             alignas(16) uint8_t val[VB];
+            PlaneExc exc[EXC_LDS];
         };
         struct Buf {
             PlaneVals<CLS, SW> v;
             Acc x[NE];
         };
+        const Shared &sh;
         const uint8_t *s_val;
         int row0, row1;  // rows of the chunk
         int slots;       // row slots in use: row0 + i TPB + tid, i < slots
@@ -44,9 +47,13 @@ template <int CLS, int SW, bool A64> struct Stencil {
         // products alternate the direction in which they walk the streamed
         // rows: the next one starts with the values that the L2 still holds
         mutable bool down = false;
+        // the chunk's listed entries
+        const PlaneExc *exc = nullptr;
+        int nexc = 0;
 
-        // Copies each thread's own rows: no barrier needed.
-        __device__ Op(const SolveArgs &A, Shared &sh, int r0, int r1) : s_val(sh.val), row0(r0), row1(r1)
+        // Copies each thread's own rows; a __syncthreads must follow for the
+        // listed entries.
+        __device__ Op(const SolveArgs &A, Shared &s, int r0, int r1) : sh(s), s_val(s.val), row0(r0), row1(r1)
         {
             const int rb = plane_row_bytes(CLS, A.pl.L), tid = threadIdx.x;
             slots = (row1 - row0 + TPB - 1) / TPB;
@@ -54,13 +61,49 @@ template <int CLS, int SW, bool A64> struct Stencil {
             const OffPtr off = off_ptr(A.off);
             edge = row0 + min(off[0], 0) < 0 || row1 - 1 + max(off[A.pl.L - 1], 0) >= A.nrows;
             const int nq = SW ? 1 : (A.pl.L + 3) >> 2;
+            if (A.nexc) {
+                auto first = [&](int r) {  // first entry of row r or later
+                    int lo = 0, hi = A.nexc;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (A.exc[mid].row < r) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    return lo;
+                };
+                const int e0 = first(row0);
+                nexc = first(row1) - e0;
+                exc = A.exc + e0;
+                if (tid < min(nexc, EXC_LDS)) s.exc[tid] = exc[tid];
+            }
             for (int i = 0; i < nlds; i++) {
                 const uint32_t r = (uint32_t)min(row0 + i * TPB + tid, row1 - 1);
                 for (int q = 0; q < nq; q++) {
                     PlaneVals<CLS, SW> v;
                     v.load(A.pl.val + (size_t)q * 4 * cls_width(CLS) * A.pl.stride, A.pl.stride, r);
-                    put(sh.val + (size_t)i * rb * TPB + (size_t)q * 4 * cls_width(CLS) * TPB, v, tid);
+                    put(s.val + (size_t)i * rb * TPB + (size_t)q * 4 * cls_width(CLS) * TPB, v, tid);
                 }
+            }
+        }
+        __device__ PlaneExc listed(int e) const
+        {
+            if (e < EXC_LDS) return sh.exc[e];
+            return exc[e];
+        }
+        // Adds the listed entries to a product that body stored at dst[i TPB +
+        // tid] as it came (the sums are Acc values, so they go on exactly where
+        // they stopped).  Beside the product's loop, which has no registers to
+        // spare for it; BiCGSTAB alone, CG folds its products into s.
+        __device__ void add_listed(double *dst, const double *g64, const float *g32) const
+        {
+            for (int e = 0; e < nexc; e++) {
+                const PlaneExc x = listed(e);
+                const int at = x.row - row0;
+                if (at % TPB != (int)threadIdx.x) continue;
+                Acc xg;
+                if constexpr (sizeof(Acc) == 8) xg = g64[x.row + x.off];
+                else xg = g32[x.row + x.off];
+                dst[at] = (double)fma_t((Acc)x.val, xg, (Acc)dst[at]);
             }
         }
         __device__ static void put(uint8_t *base, const PlaneVals<CLS, SW> &v, int t)
@@ -172,7 +215,16 @@ template <int CLS, int SW, bool A64> struct Stencil {
                                                  double (&acc)[NV]) const
         {
             if (A.use64) plane_row_f64<0, SW, NV>(A.pl64, off_ptr(A.off), (uint32_t)row, A.nrows, g, acc);
-            else plane_row_f64<CLS, SW, NV>(A.pl, off_ptr(A.off), (uint32_t)row, A.nrows, g, acc);
+            else {
+                plane_row_f64<CLS, SW, NV>(A.pl, off_ptr(A.off), (uint32_t)row, A.nrows, g, acc);
+                for (int e = 0; e < nexc; e++) {
+                    const PlaneExc x = listed(e);
+                    if (x.row == (int)row)
+#pragma unroll
+                        for (int k = 0; k < NV; k++)
+                            acc[k] = __builtin_fma((double)x.val, g[k][x.row + x.off], acc[k]);
+                }
+            }
         }
     };
 };

@@ -863,7 +863,10 @@ void Layout::release()
     if (stc) (void)hipFree(stc);
     if (blob) (void)hipFree(blob);
     if (planes) (void)hipFree(planes);
+    if (exc) (void)hipFree(exc);
     planes = nullptr;
+    exc = nullptr;
+    nexc = 0;
     planes_cls = -1;
     planes_tried = false;
     trh = nullptr;
@@ -947,6 +950,39 @@ __global__ __launch_bounds__(256) void k_planes_pack(const int *__restrict__ row
     }
 }
 
+// As k_planes_pack from the tiles, for a layout of several classes: entries of
+// class cls go to the planes, the others to the list (in any order; *n counts
+// them, cap entries are kept).
+template <int B>
+__global__ __launch_bounds__(256) void k_planes_split(const int *__restrict__ tile_ptr, int tilem,
+                                                      const int *__restrict__ tile_start,
+                                                      const int *__restrict__ tile_columnidx,
+                                                      const uint8_t *__restrict__ rowtmp, const double *__restrict__ bval,
+                                                      const uint8_t *__restrict__ bcol, const uint8_t *__restrict__ codes,
+                                                      const StencilTable *__restrict__ t, int cls, size_t stride,
+                                                      uint8_t *__restrict__ out, PlaneExc *__restrict__ exc, int cap, int *n)
+{
+    const int tr = blockIdx.x * 256 + threadIdx.x;
+    if (tr >= tilem) return;
+    const int L = t->L;
+    for (int q = tile_ptr[tr]; q < tile_ptr[tr + 1]; q++) {
+        const int c = code_to_cls(codes[q]);
+        for (int k = tile_start[q]; k < tile_start[q + 1]; k++) {
+            const int row = tr * B + rowtmp[k], off = tile_columnidx[q] * B + bcol[k] - row;
+            const double v = bval[k];
+            const float f = c == 1 ? (float)v : c == 2 ? f16_to_f32(f64_to_f16(v)) : e4m3_to_f32(f64_to_e4m3(v));
+            if (c != cls) {
+                const int e = atomicAdd(n, 1);
+                if (e < cap) exc[e] = PlaneExc{row, off, f, c};
+                continue;
+            }
+            uint8_t *p = out + plane_pos(cls, L, stride, (size_t)row, offset_pos(t, off));
+            if (cls == 1) *reinterpret_cast<float *>(p) = f;
+            else *reinterpret_cast<uint16_t *>(p) = f64_to_f16(v);
+        }
+    }
+}
+
 // Looks for the matrix's offset table: the longest row's offsets, when every
 // row is strictly ascending and draws from them.
 static int find_stencil(mf_matrix m)
@@ -968,18 +1004,65 @@ static int find_stencil(mf_matrix m)
     return MF_OK;
 }
 
+// Planes of class cls and the list of the other entries, sorted by row, class
+// and column (the order in which the slabs sum them).
+static int pack_split(mf_matrix m, Layout &L, int cls, int listed)
+{
+    hipStream_t st = stream();
+    const size_t rows = (size_t)m->tilem * m->B;
+    uint8_t *codes = nullptr;
+    int *d_n = nullptr;
+    MF_HIP(hipMallocAsync((void **)&codes, (size_t)m->tilenum + 1, st));
+    MF_HIP(hipMallocAsync((void **)&d_n, sizeof(int), st));
+    MF_HIP(hipMalloc((void **)&L.exc, sizeof(PlaneExc) * (size_t)listed));
+    MF_HIP(hipMemsetAsync(d_n, 0, sizeof(int), st));
+    int rc = classes_device(m, L.tau, L.allow_mask, codes);
+    if (rc) return rc;
+    const unsigned nb = (unsigned)((m->tilem + 255) / 256);
+#define MF_SPLIT(BB)                                                                                                    \
+    k_planes_split<BB><<<nb, 256, 0, st>>>(m->d_tile_ptr, m->tilem, m->d_tile_start, m->d_tile_columnidx, m->d_rowtmp,  \
+                                           m->d_Blockcsr_Val, m->d_Tile_csr_Col, codes, m->d_st, cls, rows, L.planes,   \
+                                           L.exc, listed, d_n)
+    if (m->B == 16) MF_SPLIT(16);
+    else if (m->B == 8) MF_SPLIT(8);
+    else MF_SPLIT(32);
+#undef MF_SPLIT
+    MF_HIP(hipGetLastError());
+    int n = 0;
+    std::vector<PlaneExc> e(listed);
+    MF_HIP(hipMemcpyAsync(&n, d_n, sizeof(int), hipMemcpyDeviceToHost, st));
+    MF_HIP(hipMemcpyAsync(e.data(), L.exc, sizeof(PlaneExc) * e.size(), hipMemcpyDeviceToHost, st));
+    MF_HIP(hipStreamSynchronize(st));
+    MF_HIP(hipFreeAsync(codes, st));
+    MF_HIP(hipFreeAsync(d_n, st));
+    if (n != listed) return fail(MF_E_FORMAT, "stencil planes: classes changed");
+    std::sort(e.begin(), e.end(), [](const PlaneExc &a, const PlaneExc &b) {
+        return a.row != b.row ? a.row < b.row : a.cls != b.cls ? a.cls < b.cls : a.off < b.off;
+    });
+    MF_HIP(upload(L.exc, e.data(), sizeof(PlaneExc) * e.size()));
+    L.nexc = n;
+    return MF_OK;
+}
+
 int ensure_planes(mf_matrix m, Layout &L)
 {
     if (L.planes_tried || !L.built) return MF_OK;
     L.planes_tried = true;
-    // one class, automatic index form
-    int cls = -1, classes = 0;
+    // automatic index form; one class, or a low-precision one and at most 1 in
+    // 1000 entries of narrower classes
+    int cls = 4, classes = 0;
+    long long nnz_cls = 0, nnz_all = 0;
     for (int code = 0; code < 5; code++)
         if (L.tiles_per_code[code] > 0) {
-            cls = code_to_cls(code);
             classes++;
+            nnz_all += L.nnz_per_code[code];
+            if (code_to_cls(code) < cls) {
+                cls = code_to_cls(code);
+                nnz_cls = L.nnz_per_code[code];
+            }
         }
-    if (classes != 1 || L.want_iw != 0 || L.split) return MF_OK;
+    const long long listed = nnz_all - nnz_cls;
+    if (!classes || (listed && (cls == 0 || listed > nnz_all / 1000)) || L.want_iw != 0 || L.split) return MF_OK;
     if (m->st_L < 0) {
         int rc = find_stencil(m);
         if (rc) return rc;
@@ -994,9 +1077,14 @@ int ensure_planes(mf_matrix m, Layout &L)
     hipStream_t st = stream();
     MF_HIP(hipMalloc((void **)&L.planes, bytes));
     MF_HIP(hipMemsetAsync(L.planes, 0, bytes, st));
-    k_planes_pack<<<(unsigned)((m->rowA + 255) / 256), 256, 0, st>>>(m->d_rowptr, m->d_col, m->d_val, m->rowA, m->d_st, cls,
-                                                                     rows, L.planes);
-    MF_HIP(hipGetLastError());
+    if (!listed) {
+        k_planes_pack<<<(unsigned)((m->rowA + 255) / 256), 256, 0, st>>>(m->d_rowptr, m->d_col, m->d_val, m->rowA, m->d_st,
+                                                                         cls, rows, L.planes);
+        MF_HIP(hipGetLastError());
+    } else {
+        int rc = pack_split(m, L, cls, (int)listed);
+        if (rc) return rc;
+    }
     L.planes_cls = cls;
     return MF_OK;
 }
