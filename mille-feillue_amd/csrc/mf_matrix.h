@@ -61,7 +61,7 @@ struct Workspace {
     unsigned long long *slots = nullptr;
     int *ctl = nullptr;
     double *out = nullptr;
-    double *r_outer = nullptr, *d = nullptr, *tmp = nullptr;
+    double *r_outer = nullptr, *d = nullptr;
     double *red = nullptr;
     // neighbour syncs of the persistent solvers, for the grid (dep_G chunks
     // of dep_trw tile rows): per chunk the other chunks whose rows its tile

@@ -80,29 +80,54 @@ __global__ void k_to_f32(const double *__restrict__ x, float *__restrict__ y, lo
     if (i < n) y[i] = (float)x[i];
 }
 
-// r = b - A x (FP64 accumulation over stored values); per-block partial ||r||^2
+// r = b - A x (FP64 accumulation over stored values); per-block partials of
+// ||r||^2 and ||b||^2 (part[block], part[blocks + block])
 template <int B, int IW>
 __global__ __launch_bounds__(256) void k_residual(DevL L, int tilem, const double *__restrict__ b,
                                                   const double *__restrict__ x, double *__restrict__ r,
                                                   double *__restrict__ part)
 {
-    __shared__ double s_w[4];
+    __shared__ double s_w[8];
     const int tr = blockIdx.x * (256 / B) + threadIdx.x / B, lane = threadIdx.x % B;
     const int lanebase = (threadIdx.x & 63) & ~(B - 1);
-    double v = 0.0;
+    double v = 0.0, vb = 0.0;
     if (tr < tilem) {
         const double *g[1] = {x};
         double acc[1] = {0.0};
         tile_row_spmv_f64<B, IW, 1>(L, tr, lane, lanebase, g, acc);
         const size_t row = (size_t)tr * B + lane;
-        const double rv = b[row] - acc[0];
+        const double bv = b[row], rv = bv - acc[0];
         r[row] = rv;
         v = rv * rv;
+        vb = bv * bv;
     }
+    v = wave_sum(v);
+    vb = wave_sum(vb);
+    if ((threadIdx.x & 63) == 0) {
+        s_w[threadIdx.x >> 6] = v;
+        s_w[4 + (threadIdx.x >> 6)] = vb;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const double *w = s_w + 4 * threadIdx.x;
+        part[threadIdx.x * gridDim.x + blockIdx.x] = ((w[0] + w[1]) + w[2]) + w[3];
+    }
+}
+
+// out[k] = sum of part[k n .. (k + 1) n), k = blockIdx.x, in a fixed order.
+__global__ __launch_bounds__(1024) void k_sum_parts(const double *__restrict__ part, int n, double *__restrict__ out)
+{
+    __shared__ double s_w[16];
+    double v = 0.0;
+    for (int i = threadIdx.x; i < n; i += 1024) v += part[(size_t)blockIdx.x * n + i];
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = ((s_w[0] + s_w[1]) + s_w[2]) + s_w[3];
+    if (threadIdx.x == 0) {
+        double s = 0.0;
+        for (int w = 0; w < 16; w++) s += s_w[w];
+        out[blockIdx.x] = s;
+    }
 }
 
 __global__ void k_axpy(double *__restrict__ x, const double *__restrict__ d, long long n)
@@ -194,7 +219,7 @@ static int ensure_ws(mf_matrix m, int G)
                  q64 = take(sizeof(double) * ncol), g32 = take(sizeof(float) * ncol * w.ring), gathered = size,
                  slots = take(sizeof(unsigned long long) * SLOT_BUFS * SLOT_WORDS * w.G), ctl = take(sizeof(int) * 8),
                  out = take(sizeof(double) * 4), r_outer = take(sizeof(double) * ncol), d = take(sizeof(double) * ncol),
-                 tmp = take(sizeof(double) * ncol), red = take(sizeof(double) * (ncol / 16 + 1024));
+                 red = take(sizeof(double) * (ncol / 16 + 1024));
     MF_HIP(hipMalloc((void **)&w.block, size));
     w.g64 = reinterpret_cast<double *>(w.block + g64);
     w.h64 = reinterpret_cast<double *>(w.block + h64);
@@ -205,7 +230,6 @@ static int ensure_ws(mf_matrix m, int G)
     w.out = reinterpret_cast<double *>(w.block + out);
     w.r_outer = reinterpret_cast<double *>(w.block + r_outer);
     w.d = reinterpret_cast<double *>(w.block + d);
-    w.tmp = reinterpret_cast<double *>(w.block + tmp);
     w.red = reinterpret_cast<double *>(w.block + red);
     // gather vectors are read up to tilen*B; entries beyond the rows stay zero
     MF_HIP(hipMemsetAsync(w.block, 0, gathered, stream()));
@@ -567,9 +591,10 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
                              rpt_out);
 }
 
-// r = b - A x over layout L; returns ||r|| (FP64) via host sum of partials.
+// r = b - A x over layout L; returns ||r|| and, if asked, ||b|| (FP64): one pass
+// over the matrix and one wait for both.
 static int residual(mf_matrix m, const Layout &L, const double *d_b, const double *d_x, double *d_r,
-                    double *norm)
+                    double *norm, double *bnorm = nullptr)
 {
     hipStream_t st = stream();
     const int B = m->B;
@@ -583,12 +608,13 @@ static int residual(mf_matrix m, const Layout &L, const double *d_b, const doubl
 #undef MF_RES_B
 #undef MF_RES
     MF_HIP(hipGetLastError());
-    std::vector<double> part(nb);
-    MF_HIP(hipMemcpyAsync(part.data(), m->ws.red, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
+    double *sums = m->ws.red + 2 * (size_t)nb, s[2];
+    k_sum_parts<<<2, 1024, 0, st>>>(m->ws.red, nb, sums);
+    MF_HIP(hipGetLastError());
+    MF_HIP(hipMemcpyAsync(s, sums, sizeof(s), hipMemcpyDeviceToHost, st));
     MF_HIP(hipStreamSynchronize(st));
-    double s = 0.0;
-    for (double v : part) s += v;
-    *norm = std::sqrt(s);
+    *norm = std::sqrt(s[0]);
+    if (bnorm) *bnorm = std::sqrt(s[1]);
     return MF_OK;
 }
 
@@ -698,10 +724,7 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     (void)hipEventDestroy(e1);
     // independent FP64 check of the returned x (outside the timed region)
     double bn = 0.0, rn = 0.0;
-    MF_HIP(hipMemsetAsync(w.tmp, 0, sizeof(double) * n, st));
-    rc = residual(m, m->L64, d_b, w.tmp, w.d, &bn);
-    if (rc) return rc;
-    rc = residual(m, m->L64, d_b, d_x, w.d, &rn);
+    rc = residual(m, m->L64, d_b, d_x, w.d, &rn, &bn);
     if (rc) return rc;
     rep->relres_true = bn > 0 ? rn / bn : rn;
     (void)relres;
