@@ -392,6 +392,11 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
         if (!finite) { finish(MF_E_NONFINITE, iter, repl, -1.0); return true; }
         if (conv || due || force) {
             // r = b - A x and s = A p on the FP64 layout; (r,r), (r,s), (p,s)
+            if (gn > 1)  // the other workgroups of the group gather x and p
+                for (size_t e = (size_t)tr0 * B * K + tid; e < (size_t)tr1 * B * K; e += TPB) {
+                    st_ag(A.x + e, A.x[e]);
+                    st_ag(A.p + e, A.p[e]);
+                }
             if (!S.allreduce(A, v, true)) return false;  // x and p of every row visible
             double t0[KLP], t1[KLP], t2[KLP];
 #pragma unroll
@@ -515,6 +520,8 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
         }
         // p, x, r updates stream the workgroup's elements [row][K] with unit
         // stride; every thread keeps one column (TPB is a multiple of K)
+        // (only r is gathered by other workgroups, where the group has any:
+        // the rest stays in the L2 instead of being written through)
         double gg[K];
         {
             const int km = tid % K;
@@ -538,10 +545,15 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
                     if (e < e1) {
                         const double pv = rv0[u] + be * pv0[u];
                         const double rv = rv0[u] - al * sv0[u];
-                        st_ag(A.p + e, pv);
-                        st_ag(A.x + e, xv0[u] + al * pv);
-                        st_ag(A.r + e, rv);
-                        if (A.haslow) st_ag(A.r32 + e, (float)rv);
+                        A.p[e] = pv;
+                        A.x[e] = xv0[u] + al * pv;
+                        if (gn > 1) {
+                            st_ag(A.r + e, rv);
+                            if (A.haslow) st_ag(A.r32 + e, (float)rv);
+                        } else {
+                            A.r[e] = rv;
+                            if (A.haslow) A.r32[e] = (float)rv;
+                        }
                         acc += rv * rv;
                     }
                 }
