@@ -21,14 +21,14 @@ template <int CLS, int SW, bool A64> struct Stencil {
         // one-workgroup solves and the reduction scratch
         static constexpr int VB = (LDS_BYTES - VECS * RPT * TPB * 8 - (RPT <= 4 ? 12 * 2048 : 0) - 1024 -
                                   EXC_LDS * (int)sizeof(PlaneExc)) / 16 * 16;
-        // rows (or quads) in flight: what the registers beside the vectors
-        // hold, at most 60 loads (the load counter holds 63) and 4 rows
-        // (two, three and four rows measure within 3 %, eight 5 % slower)
+        // rows (quads where SW = 0) in flight: two rows of 5 or 7 entries (three
+        // and four measure 0 to 4 % slower: 128^3 Poisson CG FP64 25.8 us per
+        // iteration with two, 26.8 and 26.9 with three and four; 151 x 149 x 147
+        // E4M3 24.9, 25.5, 25.5; eight 28.3), four quads, or what the registers
+        // beside the vectors hold
         static constexpr int STEP_REGS = PlaneVals<CLS, SW>::NW * (CLS == 0 ? 2 : 1) + NE * (int)sizeof(Acc) / 4;
         static constexpr int FIT = (190 - VREGS * RPT) / STEP_REGS;
-        static constexpr int LOADS = NE + (CLS == 0 ? (NE + 1) / 2 : CLS == 1 ? (NE + 2) / 4 + (NE & 1) : 1);
-        static constexpr int DLOAD = 60 / LOADS < 4 ? 60 / LOADS : 4;
-        static constexpr int DMAX = SW && RPT < DLOAD ? RPT : DLOAD;
+        static constexpr int DMAX = SW == 0 ? 4 : RPT < 2 ? RPT : 2;
         static constexpr int D = FIT < 1 ? 1 : FIT < DMAX ? FIT : DMAX;
         struct Shared {
             alignas(16) uint8_t val[VB];
