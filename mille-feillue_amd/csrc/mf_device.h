@@ -259,7 +259,7 @@ __device__ __forceinline__ int load_tcr(const DevL &L, const int *t0s, int q, in
 // flight per step: FP64 UQ64 when one row is (NB = 1), the other classes UQL4.
 // A 2000-entry row is then ~125 dependent load -> gather steps, not ~500
 // (random SPD, 1M rows: FP64 CG 315 -> 218 ms).
-template <int B, int IW, int CLS, int NR, int QS, int UQL4, int UQ64, typename AccT, typename GT>
+template <int B, int IW, int CLS, int NR, int QS, int UQL4, int UQ64, bool PF, typename AccT, typename GT>
 __device__ __forceinline__ void slab_spmv_rows(const DevL &L, const int4 *hd, const int *t0s, int q0,
                                                const int (&tcr)[NR], int row0, int r, int lanebase,
                                                const GT *__restrict__ g, AccT (&acc)[NR])
@@ -278,9 +278,15 @@ __device__ __forceinline__ void slab_spmv_rows(const DevL &L, const int4 *hd, co
             h[k] = lds_header<CLS>(hd, q0 + (kb + k) * QS);
             nqmax = max(nqmax, (h[k].y + 3) >> 2);
         }
-        for (int j0 = 0; j0 < nqmax; j0 += UQ) {
+        // The quads of one step; PF: the next step's are loaded behind this
+        // step's gathers, so a step waits for one memory latency, not two
+        // (four-byte indices, where rows are long, and where the registers
+        // allow it: random SPD 200k CG FP64 30.1 -> 29.1 us per iteration).
+        struct Step {
             Quad<CLS> v[NB][UQ];
             IdxQuad<IW> id[NB][UQ];
+        };
+        auto fetch = [&](Step &s, int j0) {
 #pragma unroll
             for (int k = 0; k < NB; k++) {
                 const int nq = (h[k].y + 3) >> 2;
@@ -291,15 +297,16 @@ __device__ __forceinline__ void slab_spmv_rows(const DevL &L, const int4 *hd, co
 #pragma unroll
                 for (int u = 0; u < UQ; u++) {
                     if (j0 + u < nq) {
-                        v[k][u].load(vals, (size_t)(j0 + u) * B + r);
-                        id[k][u].load(idx, pat ? (size_t)(j0 + u) : (size_t)(j0 + u) * B + r);
+                        s.v[k][u].load(vals, (size_t)(j0 + u) * B + r);
+                        s.id[k][u].load(idx, pat ? (size_t)(j0 + u) : (size_t)(j0 + u) * B + r);
                     } else {
-                        v[k][u].zero();
-                        id[k][u].zero();
+                        s.v[k][u].zero();
+                        s.id[k][u].zero();
                     }
                 }
             }
-            GT xg[NB][UQ][4];
+        };
+        auto gather = [&](const Step &s, GT (&xg)[NB][UQ][4]) {
 #pragma unroll
             for (int k = 0; k < NB; k++) {
                 const int t0 = 0;
@@ -314,18 +321,41 @@ __device__ __forceinline__ void slab_spmv_rows(const DevL &L, const int4 *hd, co
                 for (int u = 0; u < UQ; u++)
                     static_for<4>([&](auto e) {
                         xg[k][u][e] =
-                            ld_elem(g, gather_col<B, IW>(id[k][u].template get<e>(), tcb, t0, L, lanebase));
+                            ld_elem(g, gather_col<B, IW>(s.id[k][u].template get<e>(), tcb, t0, L, lanebase));
                     });
             }
-            // padding entries (value 0) add +0 or -0 to a sum that starts at +0
-            // and is never -0, so they leave it unchanged
+        };
+        // padding entries (value 0) add +0 or -0 to a sum that starts at +0
+        // and is never -0, so they leave it unchanged
+        auto sum = [&](const Step &s, const GT (&xg)[NB][UQ][4]) {
 #pragma unroll
             for (int k = 0; k < NB; k++)
 #pragma unroll
                 for (int u = 0; u < UQ; u++)
                     static_for<4>([&](auto e) {
-                        acc[kb + k] = fma_t((AccT)v[k][u].template get<e>(), (AccT)xg[k][u][e], acc[kb + k]);
+                        acc[kb + k] = fma_t((AccT)s.v[k][u].template get<e>(), (AccT)xg[k][u][e], acc[kb + k]);
                     });
+        };
+        if constexpr (PF) {
+            Step cur, next;
+            if (nqmax > 0) fetch(cur, 0);
+            for (int j0 = 0; j0 < nqmax; j0 += UQ) {
+                GT xg[NB][UQ][4];
+                gather(cur, xg);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(next, j0 + UQ);
+                __builtin_amdgcn_sched_barrier(0);
+                sum(cur, xg);
+                cur = next;
+            }
+        } else {
+            for (int j0 = 0; j0 < nqmax; j0 += UQ) {
+                Step s;
+                GT xg[NB][UQ][4];
+                fetch(s, j0);
+                gather(s, xg);
+                sum(s, xg);
+            }
         }
     }
 }
@@ -346,7 +376,7 @@ constexpr int CM_ACC64 = 0x10;
 // the FP32 copy of the vector (in FP64 against the FP64 vector under
 // CM_ACC64); y = a64 + (double)a32.  Only the classes in CM are read (the
 // layout holds no others).
-template <int B, int IW, int NR, int QS, int UQL4 = 2, int UQ64 = 4, int CM = CM_ALL>
+template <int B, int IW, int NR, int QS, int UQL4 = 2, int UQ64 = 4, int CM = CM_ALL, bool PF = false>
 __device__ __forceinline__ void tile_rows_spmv(const DevL &L, const int4 *hd, const int *t0s, int q0, int trq,
                                                int r, int lanebase, const double *__restrict__ g64,
                                                const float *__restrict__ g32, double (&y)[NR])
@@ -362,15 +392,15 @@ __device__ __forceinline__ void tile_rows_spmv(const DevL &L, const int4 *hd, co
         a32[k] = 0.0f;
     }
     const int row0 = trq * B + r;
-    if constexpr (CM & 1) slab_spmv_rows<B, IW, 0, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
+    if constexpr (CM & 1) slab_spmv_rows<B, IW, 0, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
     if constexpr ((CM & CM_ACC64) != 0) {
-        if constexpr (CM & 2) slab_spmv_rows<B, IW, 1, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
-        if constexpr (CM & 4) slab_spmv_rows<B, IW, 2, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
-        if constexpr (CM & 8) slab_spmv_rows<B, IW, 3, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
+        if constexpr (CM & 2) slab_spmv_rows<B, IW, 1, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
+        if constexpr (CM & 4) slab_spmv_rows<B, IW, 2, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
+        if constexpr (CM & 8) slab_spmv_rows<B, IW, 3, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g64, a64);
     } else {
-        if constexpr (CM & 2) slab_spmv_rows<B, IW, 1, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
-        if constexpr (CM & 4) slab_spmv_rows<B, IW, 2, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
-        if constexpr (CM & 8) slab_spmv_rows<B, IW, 3, NR, QS, UQL4, UQ64>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
+        if constexpr (CM & 2) slab_spmv_rows<B, IW, 1, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
+        if constexpr (CM & 4) slab_spmv_rows<B, IW, 2, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
+        if constexpr (CM & 8) slab_spmv_rows<B, IW, 3, NR, QS, UQL4, UQ64, PF>(L, hd, t0s, q0, tcr, row0, r, lanebase, g32, a32);
     }
 #pragma unroll
     for (int k = 0; k < NR; k++) y[k] = a64[k] + (double)a32[k];

@@ -431,6 +431,9 @@ template <int B, int IW, int CM = CM_ALL> struct Slabs {
     static constexpr bool lds_tags = true;  // slabs in LDS or in HBM known at compile time
     template <int TPB, int RPT, int VECS, int VREGS> struct Op {
         static constexpr int GPB = TPB / B, NR = spmv_rows(RPT, IW), TRW = RPT * GPB, LSB = lds_slab_bytes(RPT);
+        // next step's quads in flight (see slab_spmv_rows): without spills up to
+        // 4 rows per thread of CG, 2 of BiCGSTAB
+        static constexpr bool PF = IW == 4 && RPT <= (VREGS <= 4 ? 4 : 2);
         struct Shared {
             // headers of the block's tile rows, loaded once: the per-iteration
             // SpMV then issues the tile-column word and the slab loads together
@@ -465,7 +468,7 @@ template <int B, int IW, int CM = CM_ALL> struct Slabs {
 #pragma unroll 1
             for (int i0 = 0; i0 < RPT; i0 += NR) {
                 double w[NR];
-                tile_rows_spmv<B, IW, NR, GPB, UQL4, UQ64, CM>(L, sh.h, sh.t0, i0 * GPB + grp, tr0 + i0 * GPB + grp,
+                tile_rows_spmv<B, IW, NR, GPB, UQL4, UQ64, CM, PF>(L, sh.h, sh.t0, i0 * GPB + grp, tr0 + i0 * GPB + grp,
                                                                lane, lanebase, g64, g32, w);
 #pragma unroll
                 for (int k = 0; k < NR; k++)
