@@ -199,15 +199,12 @@ constexpr int RING = 4;
 
 // One allocation for all buffers of the matrix's solves (a solve of a new
 // matrix pays for it).
-static int ensure_ws(mf_matrix m, int G)
+static hipError_t alloc_ws(Workspace &w, size_t ncol, int G, int ring)
 {
-    Workspace &w = m->ws;
-    const size_t ncol = (size_t)std::max(m->tilem, m->tilen) * m->B;
-    if (w.ncol >= ncol && w.G >= G && w.block) return MF_OK;
     w.release();
     w.ncol = ncol;
     w.G = std::max(G, 1);
-    w.ring = RING;
+    w.ring = ring;
     size_t size = 0;
     auto take = [&](size_t bytes) {
         const size_t at = size;
@@ -220,7 +217,11 @@ static int ensure_ws(mf_matrix m, int G)
                  slots = take(sizeof(unsigned long long) * SLOT_BUFS * SLOT_WORDS * w.G), ctl = take(sizeof(int) * 8),
                  out = take(sizeof(double) * 4), r_outer = take(sizeof(double) * ncol), d = take(sizeof(double) * ncol),
                  red = take(sizeof(double) * (ncol / 16 + 1024));
-    MF_HIP(hipMalloc((void **)&w.block, size));
+    hipError_t e = hipMalloc((void **)&w.block, size);
+    if (e != hipSuccess) {
+        w.block = nullptr;
+        return e;
+    }
     w.g64 = reinterpret_cast<double *>(w.block + g64);
     w.h64 = reinterpret_cast<double *>(w.block + h64);
     w.q64 = reinterpret_cast<double *>(w.block + q64);
@@ -232,7 +233,18 @@ static int ensure_ws(mf_matrix m, int G)
     w.d = reinterpret_cast<double *>(w.block + d);
     w.red = reinterpret_cast<double *>(w.block + red);
     // gather vectors are read up to tilen*B; entries beyond the rows stay zero
-    MF_HIP(hipMemsetAsync(w.block, 0, gathered, stream()));
+    return hipMemsetAsync(w.block, 0, gathered, stream());
+}
+
+static int ensure_ws(mf_matrix m, int G)
+{
+    Workspace &w = m->ws;
+    const size_t ncol = (size_t)std::max(m->tilem, m->tilen) * m->B;
+    if (w.ncol >= ncol && w.G >= G && w.block) return MF_OK;
+    if (alloc_ws(w, ncol, G, RING) != hipSuccess) {
+        (void)hipGetLastError();
+        MF_HIP(alloc_ws(w, ncol, G, 1));  // short of memory: one copy
+    }
     return MF_OK;
 }
 
@@ -618,6 +630,15 @@ static int residual(mf_matrix m, const Layout &L, const double *d_b, const doubl
     return MF_OK;
 }
 
+// Whether a kernel on stencil planes exists for the rows per workgroup: up to
+// 36 rows per thread of CG, 8 of BiCGSTAB (pick_stencil_kernel).
+static bool planes_usable(mf_matrix m, const mf_opts &o)
+{
+    int G = 1, trw = 1;
+    solver_grid(m->tilem, m->B, o.grid, &G, &trw);
+    return (long long)trw * m->B <= 512ll * (o.method == MF_CG ? 36 : 8);
+}
+
 static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_opts &o, mf_report *rep)
 {
     hipStream_t st = stream();
@@ -644,9 +665,11 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     // true-residual test is final; a lossy layout either runs its passes on
     // the FP64 layout (ir_max_outer = 0) or is refined in FP64 around it
     const bool exact = !mixed || o.tau == 0.0;
-    rc = mixed ? ensure_planes(m, m->Lmix) : MF_OK;
-    if (!rc && (!mixed || !exact)) rc = ensure_planes(m, m->L64);
-    if (rc) return rc;
+    if (planes_usable(m, o)) {
+        rc = mixed ? ensure_planes(m, m->Lmix) : MF_OK;
+        if (!rc && (!mixed || !exact)) rc = ensure_planes(m, m->L64);
+        if (rc) return rc;
+    }
     rep->ms_setup = now_ms() - t0;
     rc = ensure_ws(m, std::max(1, o.grid > 0 ? o.grid : device_cu_count()));
     if (rc) return rc;

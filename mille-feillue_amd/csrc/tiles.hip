@@ -1075,7 +1075,11 @@ int ensure_planes(mf_matrix m, Layout &L)
     // most rows use a few entries of
     if (bytes > L.blob_bytes + L.blob_bytes / 4) return MF_OK;
     hipStream_t st = stream();
-    MF_HIP(hipMalloc((void **)&L.planes, bytes));
+    if (hipMalloc((void **)&L.planes, bytes) != hipSuccess) {  // short of memory: the slabs serve
+        (void)hipGetLastError();
+        L.planes = nullptr;
+        return MF_OK;
+    }
     MF_HIP(hipMemsetAsync(L.planes, 0, bytes, st));
     if (!listed) {
         k_planes_pack<<<(unsigned)((m->rowA + 255) / 256), 256, 0, st>>>(m->d_rowptr, m->d_col, m->d_val, m->rowA, m->d_st,
