@@ -62,15 +62,62 @@ __device__ __forceinline__ void st_ag(float *p, float v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// v of lane ^ 16 (HALF = 16) or lane ^ 32 added: v_permlane*_swap_b32 exchanges the
+// odd rows of 16 lanes (the upper 32 lanes) of its first operand with the even
+// rows (the lower lanes) of its second.
+template <int HALF>
+__device__ __forceinline__ double swap_add(double a, double b)
+{
+    const unsigned long long ua = (unsigned long long)__double_as_longlong(a),
+                             ub = (unsigned long long)__double_as_longlong(b);
+    unsigned r[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const unsigned x = (unsigned)(ua >> (32 * h)), y = (unsigned)(ub >> (32 * h));
+        const auto q = HALF == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
+                                  : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        r[0][h] = q[0];
+        r[1][h] = q[1];
+    }
+    auto d = [](const unsigned *w) { return __longlong_as_double((long long)((unsigned long long)w[1] << 32 | w[0])); };
+    return d(r[0]) + d(r[1]);
+}
+// Sum over the lanes of equal lane % 8, in each of them.
+__device__ __forceinline__ double column_sum(double v)
+{
+    v += dpp_row<0x128>(v);  // row_ror:8
+    v = swap_add<16>(v, v);
+    return swap_add<32>(v, v);
+}
+// Wave sums of eight values per lane at once, each step halving the values a
+// lane carries: lane l returns the sum of v[k], k = 4 bit5(l) + 2 bit4(l) + bit3(l).
+// 34 vector instructions; eight sums one after the other take about 320, a
+// microsecond of a group sync with two waves on a SIMD (48 systems x 8 columns,
+// with the poll's values side by side in the lanes: solve 26.4 -> 23.8 ms).
+__device__ __forceinline__ double wave_sum8(const double (&v)[8])
+{
+    double a[4], b[2];
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[j] = swap_add<32>(v[j], v[j + 4]);
+#pragma unroll
+    for (int j = 0; j < 2; j++) b[j] = swap_add<16>(a[j], a[j + 2]);
+    const bool odd = threadIdx.x & 8;
+    double t = (odd ? b[1] : b[0]) + dpp_row<0x128>(odd ? b[0] : b[1]);
+    t += dpp_row<0x141>(t);  // row_half_mirror: 7 - i of each 8 lanes
+    t += dpp_row<0xb1>(t);   // quad_perm 1 0 3 2
+    return t + dpp_row<0x4e>(t);  // quad_perm 2 3 0 1
+}
+
 // Group allreduce over the W workgroups of one system (a group of one only
 // reduces across its waves).  Each FP64 partial goes out as two 64-bit words
 // whose high halves carry the sync epoch and whose low halves carry one half
 // of the value each, so a word showing the current epoch holds the current
 // half whatever order the words arrive in; every workgroup of the group polls
-// the group's words until all show the epoch, lane q reading member q's words
-// (members q + 64, ... too), so one poll costs one memory latency whatever the
-// group size, and sums them in a fixed order (per lane, then a butterfly over
-// the wave: identical bits everywhere).  Two buffers alternate by epoch
+// the group's words until all show the epoch, a lane reading one value of one
+// member (of 64 lanes, eight members of eight values; further members in the
+// same lane), so one poll costs one memory latency whatever the group size, and
+// sums them in a fixed order (per lane, then over the members' lanes: identical
+// bits everywhere).  Two buffers alternate by epoch
 // parity: a buffer is rewritten only after every member has passed the next
 // sync, which it can do only after reading the buffer.
 // The epoch restarts at 0 for every task, and the sync words are cleared once
@@ -86,18 +133,16 @@ struct GroupSync {
     int gi, gn, gw0;  // index in group, group size, first workgroup of the group
     unsigned ep = 0;
 
-    // value(k), k < N: this thread's partial of sum k; the sums are left in
-    // s_bc (read them there before the next allreduce)
+    // waves(dst): leaves the wave's sums of the N values in dst[0 .. N - 1]; the
+    // group's sums are left in s_bc (read them there before the next allreduce)
     template <int N, typename F>
-    __device__ bool allreduce_f(const BatchArgs &A, F value, bool publish)
+    __device__ bool allreduce_w(const BatchArgs &A, F waves, bool publish)
     {
         static_assert(N <= BK_MAXV, "group reducer width");
+        constexpr int NV = N % 8 ? 1 : 8;  // values side by side in the lanes of a poll
+        constexpr int NC = N / NV;
         const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-#pragma unroll
-        for (int k = 0; k < N; k++) {
-            const double s = wave_sum(value(k));
-            if (lane == 0) s_red[wv * BK_MAXV + k] = s;
-        }
+        waves(s_red + wv * BK_MAXV);
         if (publish && gn > 1) __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         ++ep;
@@ -118,23 +163,24 @@ struct GroupSync {
                     __hip_atomic_store(mine + 1, tag | (bits >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 long long spins = 0;
-                double acc[N];
+                double acc[NC];
+                const int kl = lane % NV;
                 for (;;) {
                     // the abort word loads with the members' words (one latency a round)
                     const int abw = ld_agent(A.ctl);
                     bool ok = true;
 #pragma unroll
-                    for (int k = 0; k < N; k++) acc[k] = 0.0;
-                    for (int q = lane; q < gn; q += 64) {
-                        const unsigned long long *w = W + (size_t)(gw0 + q) * 2 * BK_MAXV;
+                    for (int c = 0; c < NC; c++) acc[c] = 0.0;
+                    for (int q = lane / NV; q < gn; q += 64 / NV) {
+                        const unsigned long long *w = W + (size_t)(gw0 + q) * 2 * BK_MAXV + 2 * kl;
 #pragma unroll
-                        for (int k = 0; k < N; k++) {
+                        for (int c = 0; c < NC; c++) {
                             const unsigned long long lo =
-                                __hip_atomic_load(w + 2 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                __hip_atomic_load(w + 2 * NV * c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                             const unsigned long long hi =
-                                __hip_atomic_load(w + 2 * k + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                __hip_atomic_load(w + 2 * NV * c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                             ok = ok && (lo >> 32) == ep && (hi >> 32) == ep;
-                            acc[k] += __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
+                            acc[c] += __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
                         }
                     }
                     if (__all(ok)) break;
@@ -147,9 +193,9 @@ struct GroupSync {
                     __builtin_amdgcn_s_sleep(1);
                 }
 #pragma unroll
-                for (int k = 0; k < N; k++) {
-                    const double t = wave_sum(acc[k]);
-                    if (lane == 0) s_bc[k] = t;
+                for (int c = 0; c < NC; c++) {
+                    const double t = NV == 8 ? column_sum(acc[c]) : wave_sum(acc[c]);
+                    if (lane < NV) s_bc[c * NV + lane] = t;
                 }
                 if (!ab && publish) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             }
@@ -157,6 +203,43 @@ struct GroupSync {
         }
         __syncthreads();
         return !*s_flag;
+    }
+
+    // value(k), k < N: this thread's partial of sum k
+    template <int N, typename F>
+    __device__ bool allreduce_f(const BatchArgs &A, F value, bool publish)
+    {
+        const int lane = threadIdx.x & 63;
+        return allreduce_w<N>(A, [&](double *dst) {
+            if constexpr (N % 8 == 0) {
+#pragma unroll
+                for (int c = 0; c < N; c += 8) {
+                    double v[8];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) v[k] = value(c + k);
+                    const double t = wave_sum8(v);
+                    if (lane % 8 == 0) dst[c + (lane >> 3)] = t;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < N; k++) {
+                    const double t = wave_sum(value(k));
+                    if (lane == 0) dst[k] = t;
+                }
+            }
+        }, publish);
+    }
+
+    // one partial per thread, of sum threadIdx.x % K
+    template <int K>
+    __device__ bool allreduce_col(const BatchArgs &A, double v, bool publish)
+    {
+        static_assert(K == 1 || K == 8, "column sums");
+        const int lane = threadIdx.x & 63;
+        return allreduce_w<K>(A, [&](double *dst) {
+            const double t = K == 8 ? column_sum(v) : wave_sum(v);
+            if (lane < K) dst[lane] = t;
+        }, publish);
     }
 
     template <int N>
@@ -346,23 +429,18 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
         }
     };
 
-    double v[K];
-    {
-        const int km = tid % K;
-        double acc = 0.0;
-        for (size_t e = (size_t)tr0 * B * K + tid; e < (size_t)tr1 * B * K; e += TPB) {
-            const double bv = A.b[e];
-            st_ag(A.x + e, 0.0);
-            st_ag(A.p + e, 0.0);
-            A.s[e] = 0.0;
-            st_ag(A.r + e, bv);
-            if (A.haslow) st_ag(A.r32 + e, (float)bv);
-            acc += bv * bv;
-        }
-#pragma unroll
-        for (int k = 0; k < K; k++) v[k] = k == km ? acc : 0.0;
+    // element by element, every thread keeps one column (TPB is a multiple of K)
+    double bb = 0.0;
+    for (size_t e = (size_t)tr0 * B * K + tid; e < (size_t)tr1 * B * K; e += TPB) {
+        const double bv = A.b[e];
+        st_ag(A.x + e, 0.0);
+        st_ag(A.p + e, 0.0);
+        A.s[e] = 0.0;
+        st_ag(A.r + e, bv);
+        if (A.haslow) st_ag(A.r32 + e, (float)bv);
+        bb += bv * bv;
     }
-    if (!S.allreduce(A, v, true)) return false;
+    if (!S.template allreduce_col<K>(A, bb, true)) return false;
     if (tid < K) {
         sh_b2[tid] = sh_g[tid] = sh_ref[tid] = sh.tprev[tid] = sh.bc[tid];
         sh_gp[tid] = sh_ap[tid] = 1.0;
@@ -397,7 +475,7 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
                     st_ag(A.x + e, A.x[e]);
                     st_ag(A.p + e, A.p[e]);
                 }
-            if (!S.allreduce(A, v, true)) return false;  // x and p of every row visible
+            if (!S.template allreduce_col<K>(A, 0.0, true)) return false;  // x and p of every row visible
             double t0[KLP], t1[KLP], t2[KLP];
 #pragma unroll
             for (int j = 0; j < KLP; j++) t0[j] = t1[j] = t2[j] = 0.0;
@@ -522,12 +600,11 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
         // stride; every thread keeps one column (TPB is a multiple of K)
         // (only r is gathered by other workgroups, where the group has any:
         // the rest stays in the L2 instead of being written through)
-        double gg[K];
+        double gg = 0.0;
         {
             const int km = tid % K;
             const double al = sh_al[km], be = sh_be[km];
             const size_t e1 = (size_t)tr1 * B * K;
-            double acc = 0.0;
             constexpr int U = 4;
             for (size_t e0 = (size_t)tr0 * B * K + tid; e0 < e1; e0 += (size_t)U * TPB) {
                 double rv0[U], pv0[U], xv0[U], sv0[U];
@@ -554,15 +631,13 @@ __device__ bool cg_system(const BatchArgs &A, BatchShared<K, TPB> &sh, int sys, 
                             A.r[e] = rv;
                             if (A.haslow) A.r32[e] = (float)rv;
                         }
-                        acc += rv * rv;
+                        gg += rv * rv;
                     }
                 }
             }
-#pragma unroll
-            for (int k = 0; k < K; k++) gg[k] = k == km ? acc : 0.0;
         }
         lap(1);
-        if (!S.allreduce(A, gg, true)) return false;
+        if (!S.template allreduce_col<K>(A, gg, true)) return false;
         lap(2);
         if (tid < K) {
             if (!(sh_mode[tid] & 16)) {

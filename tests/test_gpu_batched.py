@@ -188,3 +188,18 @@ def test_gpu_batched_on_chip_refusals(gpu):
     with pytest.raises(gpu.MFError):
         A.solve(np.ones(len(rp) - 1), method=gpu.MF_CG, tol=TOL, vectors=7)
     A.close()
+
+
+@pytest.mark.parametrize("nrhs", [1, 3, 8])
+@pytest.mark.parametrize("n", [500, 2100, 20000])
+def test_gpu_batched_group_sums(gpu, orc, n, nrhs):
+    # one system over two, about eight and more than 64 workgroups: the members'
+    # words of one poll fit the wave's lanes (8 members of 8 values, 64 of one)
+    # or are read in turns
+    systems = _systems(gpu, [n], seed=n)
+    b = _rhs(systems, nrhs, 5)
+    bt = gpu.Batch(systems, nrhs=nrhs, tol=TOL)
+    assert bt.info()["G"] > (64 if n == 20000 else 0)
+    xs, it, rel, rep = bt.solve([b[0][0]] if nrhs == 1 else b)
+    _check_batch(orc, systems, [b[0][0]] if nrhs == 1 else b, xs, it, rel, rep)
+    bt.close()
