@@ -93,7 +93,9 @@ __device__ __forceinline__ double column_sum(double v)
 // lane carries: lane l returns the sum of v[k], k = 4 bit5(l) + 2 bit4(l) + bit3(l).
 // 34 vector instructions; eight sums one after the other take about 320, a
 // microsecond of a group sync with two waves on a SIMD (48 systems x 8 columns,
-// with the poll's values side by side in the lanes: solve 26.4 -> 23.8 ms).
+// with the poll's values side by side in the lanes: solve 26.4 -> 23.8 ms).  The
+// eight-column kernel also needs fewer registers, 252, and so runs two workgroups
+// on a CU where it ran one (128 systems of 2000 to 20,000 rows: 226 -> 170 ms).
 __device__ __forceinline__ double wave_sum8(const double (&v)[8])
 {
     double a[4], b[2];
