@@ -50,12 +50,24 @@ struct Layout {
     void release();
 };
 
+// Entries from one copy of the published vector to the next: every copy starts
+// at a cache line of its own, in FP64 and in FP32.  The solvers' caches may keep
+// what stood beside a copy's entries in their line when they were gathered; no
+// entry of another copy may stand there (persistent.h, Reducer).
+constexpr size_t CACHE_LINE = 128;
+constexpr size_t ring_stride(size_t ncol)
+{
+    constexpr size_t per = CACHE_LINE / sizeof(float);
+    return (ncol + per - 1) / per * per;
+}
+
 // Solver scratch, sized for the matrix and grid on first use.
 struct Workspace {
     size_t ncol = 0;
     int G = 0;
     uint8_t *block = nullptr;  // the allocation behind g64 .. red
-    int ring = 1;  // copies of the published vector in g64 and g32, ncol entries apart
+    int ring = 1;        // copies of the published vector in g64 and g32
+    size_t rstride = 0;  // entries from one copy to the next: ring_stride(ncol)
     double *g64 = nullptr, *h64 = nullptr, *q64 = nullptr;
     float *g32 = nullptr;
     unsigned long long *slots = nullptr;

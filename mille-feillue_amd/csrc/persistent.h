@@ -132,7 +132,12 @@ static_assert(SYNC_K <= SLOT_WORDS, "sync line");
 // later; in between lie an allreduce that every workgroup reaches only after
 // that product, and then an invalidation by this workgroup (L1 and the XCD's
 // L2).  So no cache holds older entries when a copy is gathered again,
-// whichever workgroup of the XCD had brought them in.  That takes grid syncs:
+// whichever workgroup of the XCD had brought them in.  Caches hold lines, so
+// this takes copies that share no line (ring_stride; at 16-row tiles an odd
+// number of tile rows would otherwise start copies 1 and 3 of the FP32 vector in
+// the line of the last entries of copies 0 and 2).  Chunks may share a line:
+// it is filled by the first gather after the sync, when both chunks' entries
+// are there, and a store fills nothing but its own bytes.  And it takes grid syncs:
 // with neighbour waits every publish carries SY_ACQ, since a workgroup may read
 // (beside the entries it waits for, in the same cache line or under a value 0)
 // entries that their owner has not written yet, which another workgroup of the

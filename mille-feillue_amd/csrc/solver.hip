@@ -205,15 +205,16 @@ static hipError_t alloc_ws(Workspace &w, size_t ncol, int G, int ring)
     w.ncol = ncol;
     w.G = std::max(G, 1);
     w.ring = ring;
+    w.rstride = ring_stride(ncol);
     size_t size = 0;
-    auto take = [&](size_t bytes) {
+    auto take = [&](size_t bytes) {  // at 256 bytes: whole cache lines
         const size_t at = size;
         size += (bytes + 255) / 256 * 256;
         return at;
     };
     // the gathered vectors first: cleared below
-    const size_t g64 = take(sizeof(double) * ncol * w.ring), h64 = take(sizeof(double) * ncol),
-                 q64 = take(sizeof(double) * ncol), g32 = take(sizeof(float) * ncol * w.ring), gathered = size,
+    const size_t g64 = take(sizeof(double) * w.rstride * w.ring), h64 = take(sizeof(double) * ncol),
+                 q64 = take(sizeof(double) * ncol), g32 = take(sizeof(float) * w.rstride * w.ring), gathered = size,
                  slots = take(sizeof(unsigned long long) * SLOT_BUFS * SLOT_WORDS * w.G), ctl = take(sizeof(int) * 8),
                  out = take(sizeof(double) * 4), r_outer = take(sizeof(double) * ncol), d = take(sizeof(double) * ncol),
                  red = take(sizeof(double) * (ncol / 16 + 1024));
@@ -435,6 +436,9 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     A.g32 = w.g32;
     A.ring = w.ring;
     A.rstride = w.rstride;
+    if (w.ring > 1 && ((uintptr_t)w.g64 % CACHE_LINE || (uintptr_t)w.g32 % CACHE_LINE ||
+                       w.rstride * sizeof(float) % CACHE_LINE))
+        return fail(MF_E_ARG, "copies of the published vector share a cache line");
     A.h64 = w.h64;
     A.q64 = w.q64;
     A.slots = w.slots;
@@ -596,7 +600,7 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
         w.dep_max = ws.dep_max;
     }
     w.ring = ws.ring;
-    w.rstride = (long long)ws.ncol;
+    w.rstride = (long long)ws.rstride;
     w.vec = ws.vec;
     w.vstride = (long long)ws.ncol;
     return launch_persistent(m, L, L64, method, d_b, d_x, tol, o, G, trw, kc, w, sync, res, grid_out, block_out,
