@@ -630,7 +630,8 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                         s_s[i * TPB + tid] = acc[1];
                         publish(row, rv);
                         // registers take no running index: the FP64 copy of
-                        // the published vector hands rv over
+                        // the published vector hands rv over (A.g64 where none
+                        // is published there: only this thread touches its rows)
                         if constexpr (r_regs) {
                             if (lds || !A.has64) A.g64[row] = rv;
                         } else {
@@ -638,12 +639,15 @@ __global__ __launch_bounds__(TPB, 1) void k_cg(SolveArgs A)
                         }
                         t1[0] = fma_t(rv, rv, t1[0]);
                     }
+                if (!R.allreduce(A, t1, ring.flags(A))) return;
+                // behind the sync: a load before it would leave a neighbour
+                // chunk's entries of the line, not yet published, in the caches
+                // (chunks of 8-row tiles start in mid-line)
                 if constexpr (r_regs) {
     #pragma clang loop unroll(full)
                     for (int i = 0; i < RPT; i++)
                         if (live(i)) r_at(i) = (lds || !A.has64 ? A.g64 : ring.g64)[row_of(i)];
                 }
-                if (!R.allreduce(A, t1, ring.flags(A))) return;
                 clk.lap(4);
                 ++repl;
                 if (!isfinite(t1[0])) { finish(MF_E_NONFINITE, iter, repl, t1[0], gamma); return; }

@@ -94,3 +94,26 @@ def test_gpu_planes_beyond_register_x(gpu, orc):
             assert rep["status"] == 0 and rep["relres_true"] <= TOL and rep["streamed"] == 1
             assert abs(rep["iterations"] - sep["iterations"]) <= max(2, 0.05 * sep["iterations"])
             assert np.linalg.norm(x - y) <= 1e-8 * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("name,B,grid", [
+    ("poisson3d_33x31x29", 8, 0), ("poisson3d_33x31x29", 8, 54), ("laplace2d_97x83", 8, 16), ("band_9", 8, 9),
+    ("poisson3d_33x31x29", 32, 0), ("laplace2d_97x83", 32, 12), ("band_9", 32, 9)])
+def test_gpu_planes_replaced_residuals(gpu, orc, name, B, grid):
+    """FP64 CG whose residual is replaced every two digits, on 8- and 32-row
+    tiles, with several workgroups: chunks that start in the middle of a cache
+    line (54 workgroups of 69 tile rows of 8 rows, 16 of 63) and odd numbers of
+    tile rows.  Planes equal slabs, bit for bit."""
+    rp, ci, va = _matrix(gpu, name)
+    n = len(rp) - 1
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, n))
+    A, S = gpu.Matrix(rp, ci, va, B=B), gpu.Matrix(rp, ci, va, B=B)
+    S.set_index_width(2)
+    print(f"case {name} B={B} grid={grid}", flush=True)
+    o = dict(tol=TOL, grid=grid, rr_factor=1e-2)
+    x, rep = A.solve(b, **o)
+    y, sep = S.solve(b, **o)
+    print(f"  it={rep['iterations']} repl={rep['replacements']} grid={rep['grid']}", flush=True)
+    assert rep["status"] == 0 and rep["relres_true"] <= TOL and rep["replacements"] >= 4 and rep["grid"] > 1
+    assert (rep["iterations"], rep["replacements"], rep["grid"]) == (sep["iterations"], sep["replacements"], sep["grid"])
+    assert np.array_equal(x, y)
