@@ -138,10 +138,13 @@ static_assert(SYNC_K <= SLOT_WORDS, "sync line");
 // the line of the last entries of copies 0 and 2).  Chunks may share a line:
 // it is filled by the first gather after the sync, when both chunks' entries
 // are there, and a store fills nothing but its own bytes.  And it takes grid syncs:
-// with neighbour waits every publish carries SY_ACQ, since a workgroup may read
-// (beside the entries it waits for, in the same cache line or under a value 0)
-// entries that their owner has not written yet, which another workgroup of the
-// XCD would then find in the L2.
+// with neighbour waits there is one copy, and every publish carries SY_ACQ, since
+// a workgroup may read (beside the entries it waits for, in the same cache line
+// or under a value 0) entries that their owner has not written yet, which another
+// workgroup of the XCD would then find in the L2.  One copy alone, because what
+// is multiplied by that 0 must be finite: the allreduce of a solve's first publish
+// fills copy 0 with this solve's entries, further copies would still hold those of
+// the last solve, Inf and NaN among them when it ended so.
 // An invalidation takes the XCD's L2 about 53 ns, one after the other for its
 // workgroups (at every publish it added 1.7 us to a 2.2 us sync of 256
 // workgroups), and drops the rows that the XCD's own workgroups have just
@@ -353,7 +356,7 @@ struct RingCursor {
     // flags of the sync that follows those stores
     __device__ int flags(const SolveArgs &A) const
     {
-        return local ? 0 : slot == 0 || A.nbr ? SY_PUBLISH : SY_DRAIN;
+        return local ? 0 : slot == 0 ? SY_PUBLISH : SY_DRAIN;
     }
 };
 

@@ -457,6 +457,7 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     // BiCGSTAB's syncs after publishing p and s carry no reduction: they can
     // be neighbour waits (CG's publish sync also reduces (r, r))
     A.nbr = wants_deps(o) && w.flags && w.dep_max >= 0 && w.dep_max <= 64 ? 1 : 0;
+    if (A.nbr) A.ring = 1;  // see Reducer
     A.vec = kc.streamed && !kc.stencil ? w.vec : nullptr;
     A.vstride = w.vstride;
     if (kc.streamed && !kc.stencil && !w.vec) return fail(MF_E_ARG, "streamed kernel without its vectors");

@@ -117,3 +117,36 @@ def test_gpu_planes_replaced_residuals(gpu, orc, name, B, grid):
     assert rep["status"] == 0 and rep["relres_true"] <= TOL and rep["replacements"] >= 4 and rep["grid"] > 1
     assert (rep["iterations"], rep["replacements"], rep["grid"]) == (sep["iterations"], sep["replacements"], sep["grid"])
     assert np.array_equal(x, y)
+
+
+def test_gpu_planes_after_nonfinite_solve(gpu, orc):
+    """A solve whose published FP32 entries overflowed leaves nothing behind for
+    the next one on the same matrix: BiCGSTAB with neighbour waits, where
+    positions that hold 0 are gathered from workgroups that are not waited for
+    (the second and the fourth of four workgroups have no entry in each other's
+    rows, but an offset of the table points there)."""
+    n = 4096
+    rng = np.random.default_rng(8)
+    cols = {i: {i: -1.0 if i == n - 1 else 1.0} for i in range(n)}
+    for d in (1, 2, 2048):
+        for i in range(n - d):
+            if d < 2048 or i < 1024:
+                cols[i][i + d], cols[i + d][i] = rng.choice([-1, 1], 2) * 2.0 ** -5
+    rp = np.cumsum([0] + [len(cols[i]) for i in range(n)]).astype(np.int32)
+    ci = np.concatenate([sorted(cols[i]) for i in range(n)]).astype(np.int32)
+    va = np.concatenate([[cols[i][c] for c in sorted(cols[i])] for i in range(n)])
+    b = orc.csr_spmv(rp, ci, va, rng.uniform(-1, 1, n))
+    # (b, A b) = 2^-22 (b, b), so the first step's s exceeds FP32
+    bad = np.zeros(n)
+    bad[1500], bad[n - 1] = 2.0 ** 120 * (1 + 2.0 ** -22), 2.0 ** 120
+    o = dict(method=gpu.MF_BICGSTAB, precision=gpu.MF_MIXED, tau=0.0, rr_factor=1e-2, tol=TOL, grid=4)
+    A, F = gpu.Matrix(rp, ci, va), gpu.Matrix(rp, ci, va)
+    y, frep = F.solve(b, **o)
+    assert frep["status"] == 0 and frep["grid"] == 4 and frep["rows_per_thread"] == 2 and 0 < frep["sync_deps"] < 4
+    for turn in range(3):
+        print(f"case nonfinite, then finite, turn {turn}", flush=True)
+        _, rep = A.solve(bad, **o)
+        assert rep["status"] in (-20, -23), rep  # breakdown, non-finite sums
+        x, rep = A.solve(b, **o)
+        assert rep["status"] == 0 and rep["iterations"] == frep["iterations"]
+        assert np.array_equal(x, y)
