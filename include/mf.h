@@ -203,6 +203,13 @@ int mf_matrix_get_info(mf_matrix m, mf_matrix_info *info);
  * forms.  No reference counterpart (the reference stores four-byte columns
  * only). */
 int mf_matrix_set_index_width(mf_matrix m, int width);
+/* The stencil planes of this matrix's compute layouts: out[0] = offsets in the
+ * matrix's table (0: no stencil, or no solve has looked for one), out[1] and
+ * out[2] = class code of the planes of the FP64 and of the mixed layout (-1:
+ * none built), out[3] = entries of the mixed layout listed beside its planes,
+ * out[4] = 1 if the last solve's last launch ran on planes.  No reference
+ * counterpart. */
+int mf_matrix_planes(mf_matrix m, int out[5]);
 
 /* Precision / solver options. */
 enum { MF_CG = 0, MF_BICGSTAB = 1 };

@@ -128,7 +128,8 @@ EXPORTS = (
     "Tile_create", "Tile_destroy", "cg_solve_inc", "bicgstab", "mf_status_str", "mf_last_error",
     "mf_init", "mf_finalize", "mf_matrix_create", "mf_matrix_destroy", "mf_matrix_export", "mf_ref_tiles_free",
     "mf_matrix_encode_cols", "mf_matrix_classes", "mf_matrix_get_info", "mf_opts_default",
-    "mf_solve", "mf_solve_device", "mf_solve_device_noalloc", "mf_vendor_solve", "mf_vendor_solve_device", "mf_matrix_layout", "mf_matrix_set_index_width", "mf_spmv", "mf_spmv_bench",
+    "mf_solve", "mf_solve_device", "mf_solve_device_noalloc", "mf_vendor_solve", "mf_vendor_solve_device", "mf_matrix_layout", "mf_matrix_set_index_width",
+    "mf_matrix_planes", "mf_spmv", "mf_spmv_bench",
     "mf_solve_batched", "mf_mc_classify", "mf_memory_report", "mf_compact_rows", "mf_partition_build", "mf_free",
     "mf_gen_laplace2d", "mf_gen_poisson3d", "mf_gen_convdiff3d", "mf_gen_random_spd",
     "mf_gen_stencil_lognormal", "mf_gen_uniform", "mf_gen_normal",
@@ -169,6 +170,7 @@ def lib():
     L.mf_matrix_get_info.argtypes = [C.c_void_p, C.POINTER(Info)]
     L.mf_matrix_layout.argtypes = [C.c_void_p, C.c_double, C.c_int]
     L.mf_matrix_set_index_width.argtypes = [C.c_void_p, C.c_int]
+    L.mf_matrix_planes.argtypes = [C.c_void_p, _i]
     L.mf_spmv.argtypes = [C.c_void_p, C.c_int, _d, _d]
     L.mf_spmv_bench.argtypes = [C.c_void_p, C.c_int, C.c_int, _d]
     L.mf_opts_default.argtypes = [C.POINTER(Opts)]
@@ -406,6 +408,15 @@ class Matrix:
         """Slab index width of the compute layouts: 0 automatic, or 1, 2, 4
         bytes (that form where it fits, else the next wider one)."""
         _check(lib().mf_matrix_set_index_width(self.h, width))
+
+    def planes(self):
+        """The stencil planes built for the solves: offsets of the matrix's
+        table (0: none), class codes of the FP64 and the mixed layout's planes
+        (-1: none), entries listed beside the latter, and whether the last
+        solve ran on planes."""
+        out = np.zeros(5, np.int32)
+        _check(lib().mf_matrix_planes(self.h, _p(out, C.c_int)))
+        return dict(zip(("offsets", "fp64", "mixed", "listed", "ran"), (int(v) for v in out)))
 
     def spmv(self, x, mixed=False):
         info = self.info()

@@ -386,6 +386,20 @@ int mf_matrix_get_info(mf_matrix m, mf_matrix_info *info)
     return MF_OK;
 }
 
+int mf_matrix_planes(mf_matrix m, int out[5])
+{
+    clear_error();
+    if (!m || !out) return fail(MF_E_ARG, "null");
+    static const int code[4] = {0, 4, 3, 2};  // of each class
+    auto planes = [&](const Layout &L) { return L.built && L.planes && L.planes_cls >= 0 ? code[L.planes_cls] : -1; };
+    out[0] = std::max(0, m->st_L);
+    out[1] = planes(m->L64);
+    out[2] = planes(m->Lmix);
+    out[3] = out[2] >= 0 ? m->Lmix.nexc : 0;
+    out[4] = m->on_planes;
+    return MF_OK;
+}
+
 int mf_spmv(mf_matrix m, int mixed, const double *x, double *y)
 {
     clear_error();

@@ -112,6 +112,7 @@ struct mf_matrix_s {
     // looked for yet, 0 no stencil)
     mf::StencilTable *d_st = nullptr;
     int st_L = -1;
+    int on_planes = 0;  // the last launch of a solve ran on planes
     // compute layouts and scratch
     mf::Layout L64, Lmix;
     mf::Workspace ws;

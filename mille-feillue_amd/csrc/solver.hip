@@ -406,6 +406,7 @@ static int launch_persistent(mf_matrix m, const Layout &L, const Layout *L64, in
     A.use64 = L64 && L64 != &L ? 1 : 0;
     A.L64 = A.use64 ? L64->view(m->d_tile_ptr) : A.L;
     if (A.use64 && L64->iw != L.iw) return fail(MF_E_FORMAT, "layouts with different index forms");
+    m->on_planes = kc.stencil;
     if (kc.stencil) {
         auto view = [&](const Layout &Lv) {
             Planes P{};
@@ -1140,6 +1141,7 @@ int solve_device(mf_matrix m, const double *d_b, double *d_x, const mf_opts &o, 
     k_permute_in<<<nb, 256, 0, st>>>(m->d_perm, n, d_b, m->d_pb);
     MF_HIP(hipGetLastError());
     MF_HIP(hipEventRecord(e[1], st));
+    m->on_planes = 0;
     mf_opts oc = o;
     oc.reorder = MF_REORDER_OFF;
     int rc = solve_direct(m->child, m->d_pb, m->d_px, oc, rep);
@@ -1206,6 +1208,7 @@ int solve_noalloc(mf_matrix m, int dev, const double *d_b, double *d_x, const mf
         const unsigned nb = (unsigned)((n2 + 255) / 256);
         k_permute_in<<<nb, 256, 0, st>>>(m->d_perm, n2, d_b, m->d_pb);
         MF_HIP(hipGetLastError());
+        m->on_planes = 0;
         rc = noalloc_core(m->child, dev, m->d_pb, m->d_px, oc, rep);
         if (rc && rc != MF_E_TIMEOUT) return rc;
         const long long nx = (long long)m->tilem * m->B;

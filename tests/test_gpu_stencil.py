@@ -150,3 +150,49 @@ def test_gpu_planes_after_nonfinite_solve(gpu, orc):
         x, rep = A.solve(b, **o)
         assert rep["status"] == 0 and rep["iterations"] == frep["iterations"]
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("name,grid", [c for c in CASES if c[0] != "band_3"])
+@pytest.mark.parametrize("tau", [None, 0.0, 2.0 ** -24, 2.0 ** -11])
+def test_gpu_planes_ran(gpu, orc, name, grid, tau):
+    """The solves that the comparisons above mean to run on planes do: CG on all
+    of these grids, BiCGSTAB where its vectors fit on chip; none with an index
+    width asked for."""
+    rp, ci, va = _matrix(gpu, name)
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, len(rp) - 1))
+    A, S = gpu.Matrix(rp, ci, va), gpu.Matrix(rp, ci, va)
+    assert A.planes() == {"offsets": 0, "fp64": -1, "mixed": -1, "listed": 0, "ran": 0}
+    prec = dict(precision=gpu.MF_FP64) if tau is None else dict(precision=gpu.MF_MIXED, tau=tau, rr_factor=1e-2)
+    for method in (gpu.MF_CG, gpu.MF_BICGSTAB):
+        if method == gpu.MF_CG and name.startswith("convdiff"):
+            continue
+        print(f"case {name} grid={grid} tau={tau} method={method}", flush=True)
+        _, rep = A.solve(b, method=method, tol=TOL, grid=grid, **prec)
+        p = A.planes()
+        assert p["ran"] == (1 if method == gpu.MF_CG or rep["rows_per_thread"] > 0 else 0), (p, rep)
+        assert p["offsets"] == len({d for i in range(len(rp) - 1) for d in ci[rp[i]:rp[i + 1]] - i})
+        if p["ran"] and tau is not None:
+            assert p["mixed"] in (0, 2, 3, 4) and p["listed"] == 0
+        elif p["ran"]:
+            assert p["fp64"] == 0 and p["mixed"] == -1
+    S.solve(b, tol=TOL, index_width=2, grid=grid, **dict(prec, method=method))
+    assert S.planes() == {"offsets": 0, "fp64": -1, "mixed": -1, "listed": 0, "ran": 0}
+
+
+def test_gpu_planes_rows_per_thread(gpu, orc):
+    """17 to 36 rows per thread: the kernels of 20, 28 and 36 rows, x in the
+    caller's buffer, give the bits of the slab kernels, which stream every
+    vector there."""
+    rp, ci, va = gpu.gen_poisson3d(34, 33, 32)  # 35,904 rows on 4, 3 and 2 workgroups
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(2).uniform(-1, 1, len(rp) - 1))
+    A, S = gpu.Matrix(rp, ci, va), gpu.Matrix(rp, ci, va)
+    S.set_index_width(2)
+    for prec in (dict(precision=gpu.MF_FP64), dict(precision=gpu.MF_MIXED, tau=0.0, rr_factor=1e-4)):
+        for grid, rows in ((4, 20), (3, 28), (2, 36)):
+            print(f"case poisson3d_34x33x32 grid={grid} {prec}", flush=True)
+            x, rep = A.solve(b, tol=TOL, grid=grid, **prec)
+            y, sep = S.solve(b, tol=TOL, grid=grid, **prec)
+            assert A.planes()["ran"] == 1 and rep["rows_per_thread"] == rows and rep["streamed"] == 1
+            assert sep["rows_per_thread"] == 0 and sep["streamed"] == 1
+            assert rep["status"] == sep["status"] == 0 and rep["iterations"] == sep["iterations"]
+            assert np.array_equal(x, y)
