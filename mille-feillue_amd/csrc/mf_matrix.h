@@ -137,9 +137,15 @@ int build_reference_tiles(mf_matrix m);              // tiles.hip
 // pattern: pattern slabs where they fit (automatic index form only)
 int build_layout(mf_matrix m, Layout &L, double tau, int allow_mask, int want_iw = 0,
                  bool pattern = true);  // tiles.hip
-// the stencil planes of a built layout in the automatic index form, where the
-// matrix is a stencil and the layout holds one class (L.planes stays null
-// where not)
+// looks for the matrix's offset table, once: the longest row's offsets, when
+// every row is strictly ascending and draws from them (m->st_L)
+int find_stencil(mf_matrix m);  // tiles.hip
+// the class that planes of this layout hold, or -1: automatic index form; one
+// class, or a low-precision one and at most 1 in 1000 entries of narrower classes
+// (their number goes to listed)
+int planes_class(const Layout &L, int *listed);  // tiles.hip
+// the stencil planes of a built layout that has such a class, where the matrix
+// is a stencil (L.planes stays null where not)
 int ensure_planes(mf_matrix m, Layout &L);  // tiles.hip
 // fits bit 0: the one-byte slot form fits, bit 1: the two-byte form fits
 int index_fits(mf_matrix m, int *fits);  // tiles.hip

@@ -146,12 +146,36 @@ static int layout_cm(const Layout &L)
     return !low ? CM_F64 : e4m3_only ? CM_E4M3 : !f64 ? CM_LOW : CM_ALL;
 }
 
+// Whether planes serve a layout better than its slabs: rows per workgroup that
+// the resident plane kernels hold (up to 36 rows per thread of CG, 8 of BiCGSTAB,
+// pick_stencil_kernel), and, in solves of one workgroup, not planes of quads
+// (tables other than 5 or 7 offsets) where the slabs are in LDS with up to two rows
+// per thread, nor with more rows in FP64 on more than 8 offsets or BiCGSTAB on
+// FP16.  There every product waits for LDS alone, and the slabs' loop has two
+// rows' quads in flight; measured, planes / slabs, ms: 27-point BiCGSTAB of 512 rows
+// FP64 0.238 / 0.195, 729 rows FP16 0.531 / 0.407, 1728 rows FP64 0.687 / 0.602;
+// 3 offsets, 1000 rows, CG 0.199 / 0.166; on the other side, slabs too long for
+// LDS: 13 offsets, 1000 rows, FP64 BiCGSTAB 0.87 of the slabs' time, 9 offsets, 2000
+// rows, FP32 CG 0.84; 3 offsets, 2000 rows, FP64 CG 0.92.
+static bool planes_serve(mf_matrix m, const Layout &L, int method, long long rows_per_wg, int G)
+{
+    int listed = 0;
+    const int cls = planes_class(L, &listed);
+    if (cls < 0 || m->st_L <= 0) return false;
+    const int q = (int)((rows_per_wg + 511) / 512);
+    if (q > (method == MF_CG ? 36 : 8)) return false;
+    if (G > 1 || plane_sw(m->st_L) || q > 4) return true;
+    if (q <= 2) return L.blob_bytes > (unsigned long long)lds_slab_bytes(std::max(1, q));
+    return !(cls == 0 && m->st_L > 8) && !(cls == 2 && method == MF_BICGSTAB);
+}
+
 // The kernel on a layout's stencil planes (and, when the passes read the FP64
-// layout, on its planes too); none where they are missing or a workgroup's
-// rows exceed the resident kernels.
+// layout, on its planes too); none where they are missing or the slabs serve
+// better.
 static KernelChoice pick_stencil(mf_matrix m, const Layout &L, const Layout *L64, int method, long long rows_per_wg, int G)
 {
     if (!L.planes || (L64 && L64 != &L && !L64->planes)) return KernelChoice{};
+    if (!planes_serve(m, L, method, rows_per_wg, G)) return KernelChoice{};
     if (L.nexc && method == MF_CG) return KernelChoice{};  // see add_listed
     KernelChoice k;
     switch (L.planes_cls) {
@@ -636,13 +660,15 @@ static int residual(mf_matrix m, const Layout &L, const double *d_b, const doubl
     return MF_OK;
 }
 
-// Whether a kernel on stencil planes exists for the rows per workgroup: up to
-// 36 rows per thread of CG, 8 of BiCGSTAB (pick_stencil_kernel).
-static bool planes_usable(mf_matrix m, const mf_opts &o)
+// Builds the planes of a layout that a solve with these options runs on.
+static int ensure_serving_planes(mf_matrix m, Layout &L, const mf_opts &o)
 {
-    int G = 1, trw = 1;
+    int G = 1, trw = 1, listed = 0;
+    if (planes_class(L, &listed) < 0) return MF_OK;
+    int rc = find_stencil(m);
+    if (rc) return rc;
     solver_grid(m->tilem, m->B, o.grid, &G, &trw);
-    return (long long)trw * m->B <= 512ll * (o.method == MF_CG ? 36 : 8);
+    return planes_serve(m, L, o.method, (long long)trw * m->B, G) ? ensure_planes(m, L) : MF_OK;
 }
 
 static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_opts &o, mf_report *rep)
@@ -671,11 +697,10 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     // true-residual test is final; a lossy layout either runs its passes on
     // the FP64 layout (ir_max_outer = 0) or is refined in FP64 around it
     const bool exact = !mixed || o.tau == 0.0;
-    if (planes_usable(m, o)) {
-        rc = mixed ? ensure_planes(m, m->Lmix) : MF_OK;
-        if (!rc && (!mixed || !exact)) rc = ensure_planes(m, m->L64);
-        if (rc) return rc;
-    }
+    rc = ensure_serving_planes(m, mixed ? m->Lmix : m->L64, o);
+    // the passes of a lossy layout on planes read the FP64 layout's
+    if (!rc && !exact && m->Lmix.planes) rc = ensure_planes(m, m->L64);
+    if (rc) return rc;
     rep->ms_setup = now_ms() - t0;
     rc = ensure_ws(m, std::max(1, o.grid > 0 ? o.grid : device_cu_count()));
     if (rc) return rc;
@@ -738,6 +763,8 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     int fallback = 0;
     if (!exact && (status == MF_E_DIVERGED || status == MF_E_BREAKDOWN || status == MF_E_NONFINITE ||
                    status == MF_E_MAXIT)) {
+        rc = ensure_serving_planes(m, m->L64, o);
+        if (rc) return rc;
         rc = launch_inner(m, m->L64, nullptr, o.method, d_b, d_x, o.tol, o, true, &ir, &G, &TPB, &RPT);
         if (rc) return rc;
         status = ir.status;

@@ -983,10 +983,9 @@ __global__ __launch_bounds__(256) void k_planes_split(const int *__restrict__ ti
     }
 }
 
-// Looks for the matrix's offset table: the longest row's offsets, when every
-// row is strictly ascending and draws from them.
-static int find_stencil(mf_matrix m)
+int find_stencil(mf_matrix m)
 {
+    if (m->st_L >= 0) return MF_OK;
     m->st_L = 0;
     if (m->rowA != m->colA || !m->nnz || m->d_split) return MF_OK;
     hipStream_t st = stream();
@@ -1044,12 +1043,8 @@ static int pack_split(mf_matrix m, Layout &L, int cls, int listed)
     return MF_OK;
 }
 
-int ensure_planes(mf_matrix m, Layout &L)
+int planes_class(const Layout &L, int *listed_out)
 {
-    if (L.planes_tried || !L.built) return MF_OK;
-    L.planes_tried = true;
-    // automatic index form; one class, or a low-precision one and at most 1 in
-    // 1000 entries of narrower classes
     int cls = 4, classes = 0;
     long long nnz_cls = 0, nnz_all = 0;
     for (int code = 0; code < 5; code++)
@@ -1062,12 +1057,20 @@ int ensure_planes(mf_matrix m, Layout &L)
             }
         }
     const long long listed = nnz_all - nnz_cls;
-    if (!classes || (listed && (cls == 0 || listed > nnz_all / 1000)) || L.want_iw != 0 || L.split) return MF_OK;
-    if (m->st_L < 0) {
-        int rc = find_stencil(m);
-        if (rc) return rc;
-    }
-    if (!m->st_L) return MF_OK;
+    *listed_out = (int)listed;
+    if (!classes || (listed && (cls == 0 || listed > nnz_all / 1000)) || L.want_iw != 0 || L.split) return -1;
+    return cls;
+}
+
+int ensure_planes(mf_matrix m, Layout &L)
+{
+    if (L.planes_tried || !L.built) return MF_OK;
+    L.planes_tried = true;
+    int listed = 0;
+    const int cls = planes_class(L, &listed);
+    if (cls < 0) return MF_OK;
+    int rc = find_stencil(m);
+    if (rc || !m->st_L) return rc;
     const size_t rows = (size_t)m->tilem * m->B;
     const size_t bytes = rows * plane_row_bytes(cls, m->st_L);
     // planes hold a value for every row and offset: worth it where that is
@@ -1086,7 +1089,7 @@ int ensure_planes(mf_matrix m, Layout &L)
                                                                          cls, rows, L.planes);
         MF_HIP(hipGetLastError());
     } else {
-        int rc = pack_split(m, L, cls, (int)listed);
+        rc = pack_split(m, L, cls, listed);
         if (rc) return rc;
     }
     L.planes_cls = cls;

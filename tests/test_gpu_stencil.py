@@ -196,3 +196,29 @@ def test_gpu_planes_rows_per_thread(gpu, orc):
             assert sep["rows_per_thread"] == 0 and sep["streamed"] == 1
             assert rep["status"] == sep["status"] == 0 and rep["iterations"] == sep["iterations"]
             assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("name,tau,method,ran", [
+    ("laplace2d_30x31", None, 0, 1), ("laplace2d_30x31", 2.0 ** -11, 1, 1),
+    ("band_3", None, 0, 0), ("band_3", 2.0 ** -11, 1, 0),
+    ("convdiff_8", None, 1, 0), ("convdiff_9", 2.0 ** -24, 1, 0), ("convdiff_9", None, 1, 1), ("convdiff_12", None, 1, 0),
+    ("convdiff_12", 2.0 ** -24, 1, 1), ("convdiff_12", 2.0 ** -11, 1, 0),
+    ("band_9_2000", None, 0, 0), ("band_9_2000", 2.0 ** -24, 0, 1), ("band_9_2000", 2.0 ** -11, 0, 1)])
+def test_gpu_planes_one_workgroup(gpu, orc, name, tau, method, ran):
+    """One workgroup runs planes of quads only where they are faster than its
+    slabs (planes_serve in solver.hip), with the bits of the slabs either way."""
+    if name.startswith("convdiff"):
+        rp, ci, va = gpu.gen_convdiff3d(int(name.split("_")[1]), 10.0, 1.0, 0)
+    else:
+        rp, ci, va = _banded(2000, (1, 7, 40, 41), np.random.default_rng(5)) if name == "band_9_2000" else _matrix(gpu, name)
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, len(rp) - 1))
+    A, S = gpu.Matrix(rp, ci, va), gpu.Matrix(rp, ci, va)
+    S.set_index_width(2)
+    prec = dict(precision=gpu.MF_FP64) if tau is None else dict(precision=gpu.MF_MIXED, tau=tau, rr_factor=1e-2)
+    print(f"case {name} tau={tau} method={method}", flush=True)
+    x, rep = A.solve(b, method=method, tol=TOL, **prec)
+    y, sep = S.solve(b, method=method, tol=TOL, **prec)
+    print(f"  it={rep['iterations']} rpt={rep['rows_per_thread']} {A.planes()}", flush=True)
+    assert rep["grid"] == 1 and rep["status"] == 0 and rep["relres_true"] <= TOL
+    assert A.planes()["ran"] == ran
+    assert rep["iterations"] == sep["iterations"] and np.array_equal(x, y)
