@@ -252,11 +252,13 @@ typedef struct {
                            more than 64); MF_SYNC_GLOBAL: a grid barrier */
     int vectors;        /* MF_VECTORS_AUTO (default): the Krylov vectors of a
                            workgroup's rows stay in registers and LDS where they
-                           fit (CG up to 16 rows per thread at B >= 16, else 8;
-                           BiCGSTAB 8) and are streamed from HBM beyond that;
+                           fit (CG up to 16 rows per thread at B >= 16 and on
+                           stencil planes, else 8; BiCGSTAB 8) and are streamed
+                           from HBM beyond that (CG on planes, up to 36 rows per
+                           thread: x alone);
                            MF_VECTORS_HBM: single systems: MF_E_UNSUPPORTED where
-                           the vectors fit on chip (forcing the streamed kernels
-                           there is switched off);
+                           the slab kernels hold the vectors on chip (forcing the
+                           streamed kernels there is switched off);
                            MF_VECTORS_ONCHIP: single systems: MF_E_UNSUPPORTED
                            where they do not fit on chip.
                            Batches: AUTO and HBM keep the vectors in HBM (one

@@ -591,6 +591,9 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
     int G = 1, trw = 1;
     solver_grid(m->tilem, m->B, o.grid, &G, &trw);
     KernelChoice kc = pick_stencil(m, L, L64, method, (long long)trw * m->B, G);
+    // vectors in HBM asked for: the slab kernels stream from 9 rows per thread on
+    // at 8-row tiles, where the planes' kernels still hold them
+    if (o.vectors == MF_VECTORS_HBM && !kc.streamed) kc = KernelChoice{};
     if (!kc.fn) kc = pick(m->B, L.iw, method, (long long)trw * m->B, false, layout_cm(L), G);
     if (!kc.fn) return fail(MF_E_UNSUPPORTED, "no persistent kernel for this tile size and index form");
     // streaming the vectors of a system whose rows fit on chip is switched

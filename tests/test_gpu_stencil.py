@@ -222,3 +222,20 @@ def test_gpu_planes_one_workgroup(gpu, orc, name, tau, method, ran):
     assert rep["grid"] == 1 and rep["status"] == 0 and rep["relres_true"] <= TOL
     assert A.planes()["ran"] == ran
     assert rep["iterations"] == sep["iterations"] and np.array_equal(x, y)
+
+
+def test_gpu_hbm_vectors_beyond_the_slab_kernels(gpu, orc):
+    """9 to 16 rows per thread on 8-row tiles: CG on planes holds the vectors,
+    the slab kernels stream them, and vectors = MF_VECTORS_HBM is served by those,
+    with the same bits."""
+    rp, ci, va = gpu.gen_poisson3d(34, 33, 32)
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(2).uniform(-1, 1, len(rp) - 1))
+    A = gpu.Matrix(rp, ci, va, B=8)
+    print("case poisson3d_34x33x32 B=8 grid=5", flush=True)
+    x, rep = A.solve(b, tol=TOL, grid=5)
+    assert rep["status"] == 0 and rep["streamed"] == 0 and rep["rows_per_thread"] == 16 and A.planes()["ran"] == 1
+    y, sep = A.solve(b, tol=TOL, grid=5, vectors=gpu.MF_VECTORS_HBM)
+    assert sep["status"] == 0 and sep["streamed"] == 1 and A.planes()["ran"] == 0
+    assert rep["iterations"] == sep["iterations"] and np.array_equal(x, y)
+    with pytest.raises(gpu.MFError):  # 8 rows per thread: the slab kernels hold them
+        A.solve(b, tol=TOL, grid=9, vectors=gpu.MF_VECTORS_HBM)
