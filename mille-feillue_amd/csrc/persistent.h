@@ -1462,14 +1462,16 @@ template <class M> KernelChoice pick_stencil_acc64(int method, long long rows_pe
     k.acc64 = 1;
     return k;
 }
-template <int CLS> KernelChoice pick_stencil_class(int L, int method, long long rows_per_wg, int G)
+// sum64: small systems (pick_stencil_acc64) sum low-precision values in FP64.
+template <int CLS> KernelChoice pick_stencil_class(int L, int method, long long rows_per_wg, int G, bool sum64)
 {
     const int sw = plane_sw(L);
     KernelChoice k;
     if constexpr (CLS > 0) {
-        k = sw == 5   ? pick_stencil_acc64<Stencil<CLS, 5, true>>(method, rows_per_wg, G)
-            : sw == 7 ? pick_stencil_acc64<Stencil<CLS, 7, true>>(method, rows_per_wg, G)
-                      : pick_stencil_acc64<Stencil<CLS, 0, true>>(method, rows_per_wg, G);
+        if (sum64)
+            k = sw == 5   ? pick_stencil_acc64<Stencil<CLS, 5, true>>(method, rows_per_wg, G)
+                : sw == 7 ? pick_stencil_acc64<Stencil<CLS, 7, true>>(method, rows_per_wg, G)
+                          : pick_stencil_acc64<Stencil<CLS, 0, true>>(method, rows_per_wg, G);
         if (k.fn) return k;
     }
     return sw == 5   ? pick_stencil_kernel<Stencil<CLS, 5, false>>(method, rows_per_wg)
@@ -1477,10 +1479,10 @@ template <int CLS> KernelChoice pick_stencil_class(int L, int method, long long 
                      : pick_stencil_kernel<Stencil<CLS, 0, false>>(method, rows_per_wg);
 }
 // one class each: solver_st64.hip, solver_st32.hip, solver_st16.hip, solver_st8.hip
-KernelChoice pick_stencil_f64(int L, int method, long long rows_per_wg, int G);
-KernelChoice pick_stencil_f32(int L, int method, long long rows_per_wg, int G);
-KernelChoice pick_stencil_f16(int L, int method, long long rows_per_wg, int G);
-KernelChoice pick_stencil_e4m3(int L, int method, long long rows_per_wg, int G);
+KernelChoice pick_stencil_f64(int L, int method, long long rows_per_wg, int G, bool sum64);
+KernelChoice pick_stencil_f32(int L, int method, long long rows_per_wg, int G, bool sum64);
+KernelChoice pick_stencil_f16(int L, int method, long long rows_per_wg, int G, bool sum64);
+KernelChoice pick_stencil_e4m3(int L, int method, long long rows_per_wg, int G, bool sum64);
 
 // tile sizes and class masks instantiated in their own translation units
 KernelChoice pick_b8(int iw, int method, long long rows_per_wg, bool stream);   // solver_b8.hip

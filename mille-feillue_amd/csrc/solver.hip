@@ -177,12 +177,15 @@ static KernelChoice pick_stencil(mf_matrix m, const Layout &L, const Layout *L64
     if (!L.planes || (L64 && L64 != &L && !L64->planes)) return KernelChoice{};
     if (!planes_serve(m, L, method, rows_per_wg, G)) return KernelChoice{};
     if (L.nexc && method == MF_CG) return KernelChoice{};  // see add_listed
+    // low-precision values summed in FP64 where the slabs' are (see pick), so
+    // that the two agree bit for bit: 16-row tiles
+    const bool sum64 = m->B == 16;
     KernelChoice k;
     switch (L.planes_cls) {
-    case 0: k = pick_stencil_f64(m->st_L, method, rows_per_wg, G); break;
-    case 1: k = pick_stencil_f32(m->st_L, method, rows_per_wg, G); break;
-    case 2: k = pick_stencil_f16(m->st_L, method, rows_per_wg, G); break;
-    case 3: k = pick_stencil_e4m3(m->st_L, method, rows_per_wg, G); break;
+    case 0: k = pick_stencil_f64(m->st_L, method, rows_per_wg, G, sum64); break;
+    case 1: k = pick_stencil_f32(m->st_L, method, rows_per_wg, G, sum64); break;
+    case 2: k = pick_stencil_f16(m->st_L, method, rows_per_wg, G, sum64); break;
+    case 3: k = pick_stencil_e4m3(m->st_L, method, rows_per_wg, G, sum64); break;
     }
     k.stencil = k.fn ? 1 : 0;
     return k;

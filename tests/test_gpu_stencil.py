@@ -239,3 +239,32 @@ def test_gpu_hbm_vectors_beyond_the_slab_kernels(gpu, orc):
     assert rep["iterations"] == sep["iterations"] and np.array_equal(x, y)
     with pytest.raises(gpu.MFError):  # 8 rows per thread: the slab kernels hold them
         A.solve(b, tol=TOL, grid=9, vectors=gpu.MF_VECTORS_HBM)
+
+
+@pytest.mark.parametrize("name,grid", [
+    ("laplace2d_30x31", 0), ("laplace2d_97x83", 0), ("laplace2d_97x83", 3), ("poisson3d_33x31x29", 0),
+    ("poisson3d_33x31x29", 19), ("convdiff_14", 0), ("convdiff_21", 5), ("lognormal_3d", 0), ("band_9", 0), ("band_31", 0)])
+@pytest.mark.parametrize("B", [8, 32])
+@pytest.mark.parametrize("tau", [None, 0.0, 2.0 ** -24, 2.0 ** -11])
+def test_gpu_planes_equal_slabs_tile_sizes(gpu, orc, name, grid, B, tau):
+    """8- and 32-row tiles: planes and slabs sum low-precision values alike (in
+    FP32 at every size), so iterations and x agree bit for bit; CG with entries
+    listed beside the planes stays on the slabs."""
+    rp, ci, va = _matrix(gpu, name)
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, len(rp) - 1))
+    A, S = gpu.Matrix(rp, ci, va, B=B), gpu.Matrix(rp, ci, va, B=B)
+    S.set_index_width(2)
+    prec = dict(precision=gpu.MF_FP64) if tau is None else dict(precision=gpu.MF_MIXED, tau=tau, rr_factor=1e-2)
+    for method in (gpu.MF_CG, gpu.MF_BICGSTAB):
+        if method == gpu.MF_CG and name.startswith("convdiff"):
+            continue
+        o = dict(method=method, tol=TOL, grid=grid, **prec)
+        print(f"case {name} B={B} grid={grid} tau={tau} method={method}", flush=True)
+        x, rep = A.solve(b, **o)
+        p = A.planes()
+        y, sep = S.solve(b, **o)
+        print(f"  it={rep['iterations']} slabs {sep['iterations']} rpt={rep['rows_per_thread']} {p}", flush=True)
+        assert rep["status"] == 0 and rep["relres_true"] <= TOL, rep
+        assert p["ran"] == (0 if p["listed"] and method == gpu.MF_CG else 1)
+        assert (rep["iterations"], rep["replacements"], rep["grid"]) == (sep["iterations"], sep["replacements"], sep["grid"])
+        assert np.array_equal(x, y)
