@@ -206,7 +206,8 @@ int mf_matrix_set_index_width(mf_matrix m, int width);
 /* The stencil planes of this matrix's compute layouts: out[0] = offsets in the
  * matrix's table (0: no stencil, or no solve has looked for one), out[1] and
  * out[2] = class code of the planes of the FP64 and of the mixed layout (-1:
- * none built), out[3] = entries of the mixed layout listed beside its planes,
+ * none built), out[3] = entries of the mixed layout that its planes list (CG
+ * runs on the slabs where there are any, and does not build such planes),
  * out[4] = 1 if the last solve's last launch ran on planes.  No reference
  * counterpart. */
 int mf_matrix_planes(mf_matrix m, int out[5]);

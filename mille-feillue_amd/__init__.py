@@ -412,7 +412,7 @@ class Matrix:
     def planes(self):
         """The stencil planes built for the solves: offsets of the matrix's
         table (0: none), class codes of the FP64 and the mixed layout's planes
-        (-1: none), entries listed beside the latter, and whether the last
+        (-1: none), entries that the latter list, and whether the last
         solve ran on planes."""
         out = np.zeros(5, np.int32)
         _check(lib().mf_matrix_planes(self.h, _p(out, C.c_int)))

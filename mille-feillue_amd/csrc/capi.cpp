@@ -393,9 +393,10 @@ int mf_matrix_planes(mf_matrix m, int out[5])
     static const int code[4] = {0, 4, 3, 2};  // of each class
     auto planes = [&](const Layout &L) { return L.built && L.planes && L.planes_cls >= 0 ? code[L.planes_cls] : -1; };
     out[0] = std::max(0, m->st_L);
+    out[3] = 0;
     out[1] = planes(m->L64);
     out[2] = planes(m->Lmix);
-    out[3] = out[2] >= 0 ? m->Lmix.nexc : 0;
+    if (m->Lmix.built && m->st_L > 0 && planes_class(m->Lmix, &out[3]) < 0) out[3] = 0;
     out[4] = m->on_planes;
     return MF_OK;
 }

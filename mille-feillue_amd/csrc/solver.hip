@@ -148,7 +148,7 @@ static int layout_cm(const Layout &L)
 
 // Whether planes serve a layout better than its slabs: rows per workgroup that
 // the resident plane kernels hold (up to 36 rows per thread of CG, 8 of BiCGSTAB,
-// pick_stencil_kernel), and, in solves of one workgroup, not planes of quads
+// pick_stencil_kernel), no listed entries in CG, and, in solves of one workgroup, not planes of quads
 // (tables other than 5 or 7 offsets) where the slabs are in LDS with up to two rows
 // per thread, nor with more rows in FP64 on more than 8 offsets or BiCGSTAB on
 // FP16.  There every product waits for LDS alone, and the slabs' loop has two
@@ -163,7 +163,7 @@ static bool planes_serve(mf_matrix m, const Layout &L, int method, long long row
     const int cls = planes_class(L, &listed);
     if (cls < 0 || m->st_L <= 0) return false;
     const int q = (int)((rows_per_wg + 511) / 512);
-    if (q > (method == MF_CG ? 36 : 8)) return false;
+    if (q > (method == MF_CG ? 36 : 8) || (listed && method == MF_CG)) return false;  // CG: see add_listed
     if (G > 1 || plane_sw(m->st_L) || q > 4) return true;
     if (q <= 2) return L.blob_bytes > (unsigned long long)lds_slab_bytes(std::max(1, q));
     return !(cls == 0 && m->st_L > 8) && !(cls == 2 && method == MF_BICGSTAB);
@@ -176,7 +176,6 @@ static KernelChoice pick_stencil(mf_matrix m, const Layout &L, const Layout *L64
 {
     if (!L.planes || (L64 && L64 != &L && !L64->planes)) return KernelChoice{};
     if (!planes_serve(m, L, method, rows_per_wg, G)) return KernelChoice{};
-    if (L.nexc && method == MF_CG) return KernelChoice{};  // see add_listed
     // low-precision values summed in FP64 where the slabs' are (see pick), so
     // that the two agree bit for bit: 16-row tiles
     const bool sum64 = m->B == 16;
@@ -666,15 +665,18 @@ static int residual(mf_matrix m, const Layout &L, const double *d_b, const doubl
     return MF_OK;
 }
 
-// Builds the planes of a layout that a solve with these options runs on.
-static int ensure_serving_planes(mf_matrix m, Layout &L, const mf_opts &o)
+// Builds the planes that a solve with these options runs on: the layout's, and,
+// where its true-residual passes read the FP64 layout L64, that one's.
+static int ensure_serving_planes(mf_matrix m, Layout &L, Layout *L64, const mf_opts &o)
 {
     int G = 1, trw = 1, listed = 0;
     if (planes_class(L, &listed) < 0) return MF_OK;
     int rc = find_stencil(m);
     if (rc) return rc;
     solver_grid(m->tilem, m->B, o.grid, &G, &trw);
-    return planes_serve(m, L, o.method, (long long)trw * m->B, G) ? ensure_planes(m, L) : MF_OK;
+    if (!planes_serve(m, L, o.method, (long long)trw * m->B, G)) return MF_OK;
+    rc = ensure_planes(m, L);
+    return rc || !L.planes || !L64 ? rc : ensure_planes(m, *L64);
 }
 
 static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_opts &o, mf_report *rep)
@@ -703,9 +705,7 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     // true-residual test is final; a lossy layout either runs its passes on
     // the FP64 layout (ir_max_outer = 0) or is refined in FP64 around it
     const bool exact = !mixed || o.tau == 0.0;
-    rc = ensure_serving_planes(m, mixed ? m->Lmix : m->L64, o);
-    // the passes of a lossy layout on planes read the FP64 layout's
-    if (!rc && !exact && m->Lmix.planes) rc = ensure_planes(m, m->L64);
+    rc = ensure_serving_planes(m, mixed ? m->Lmix : m->L64, exact ? nullptr : &m->L64, o);
     if (rc) return rc;
     rep->ms_setup = now_ms() - t0;
     rc = ensure_ws(m, std::max(1, o.grid > 0 ? o.grid : device_cu_count()));
@@ -769,7 +769,7 @@ static int solve_direct(mf_matrix m, const double *d_b, double *d_x, const mf_op
     int fallback = 0;
     if (!exact && (status == MF_E_DIVERGED || status == MF_E_BREAKDOWN || status == MF_E_NONFINITE ||
                    status == MF_E_MAXIT)) {
-        rc = ensure_serving_planes(m, m->L64, o);
+        rc = ensure_serving_planes(m, m->L64, nullptr, o);
         if (rc) return rc;
         rc = launch_inner(m, m->L64, nullptr, o.method, d_b, d_x, o.tol, o, true, &ir, &G, &TPB, &RPT);
         if (rc) return rc;

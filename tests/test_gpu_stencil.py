@@ -268,3 +268,20 @@ def test_gpu_planes_equal_slabs_tile_sizes(gpu, orc, name, grid, B, tau):
         assert p["ran"] == (0 if p["listed"] and method == gpu.MF_CG else 1)
         assert (rep["iterations"], rep["replacements"], rep["grid"]) == (sep["iterations"], sep["replacements"], sep["grid"])
         assert np.array_equal(x, y)
+
+
+def test_gpu_planes_with_listed_entries(gpu, orc):
+    """A rounded layout with a few tiles of a narrower class (lognormal stencil, FP16
+    tiles of 8 rows, 62 entries in E4M3): CG, which runs on its slabs, builds no
+    planes for it; BiCGSTAB builds them and runs on them, and CG still does not."""
+    rp, ci, va = _matrix(gpu, "lognormal_3d")
+    b = orc.csr_spmv(rp, ci, va, np.random.default_rng(1).uniform(-1, 1, len(rp) - 1))
+    A = gpu.Matrix(rp, ci, va, B=8)
+    o = dict(tol=TOL, precision=gpu.MF_MIXED, tau=2.0 ** -11, rr_factor=1e-2)
+    x, rep = A.solve(b, method=gpu.MF_CG, **o)
+    assert rep["status"] == 0 and rep["fallback"] == 0
+    assert A.planes() == {"offsets": 7, "fp64": -1, "mixed": -1, "listed": 62, "ran": 0}
+    _, rep2 = A.solve(b, method=gpu.MF_BICGSTAB, **o)
+    assert rep2["status"] == 0 and A.planes() == {"offsets": 7, "fp64": 0, "mixed": 3, "listed": 62, "ran": 1}
+    y, rep3 = A.solve(b, method=gpu.MF_CG, **o)
+    assert A.planes()["ran"] == 0 and rep3["iterations"] == rep["iterations"] and np.array_equal(x, y)
