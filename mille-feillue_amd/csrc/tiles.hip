@@ -990,7 +990,12 @@ int find_stencil(mf_matrix m)
     if (m->rowA != m->colA || !m->nnz || m->d_split) return MF_OK;
     hipStream_t st = stream();
     const unsigned nb = (unsigned)((m->rowA + 255) / 256);
-    if (!m->d_st) MF_HIP(hipMalloc((void **)&m->d_st, sizeof(StencilTable)));
+    if (!m->d_st && hipMalloc((void **)&m->d_st, sizeof(StencilTable)) != hipSuccess) {
+        (void)hipGetLastError();  // short of memory: the slabs serve
+        m->d_st = nullptr;
+        m->st_L = -1;
+        return MF_OK;
+    }
     MF_HIP(hipMemsetAsync(m->d_st, 0, sizeof(StencilTable), st));
     k_longest_row<<<nb, 256, 0, st>>>(m->d_rowptr, m->rowA, &m->d_st->key);
     k_stencil_table<<<1, 64, 0, st>>>(m->d_rowptr, m->d_col, m->rowA, m->d_st);
@@ -1004,37 +1009,45 @@ int find_stencil(mf_matrix m)
 }
 
 // Planes of class cls and the list of the other entries, sorted by row, class
-// and column (the order in which the slabs sum them).
+// and column (the order in which the slabs sum them).  MF_E_NOMEM when an
+// allocation fails.
 static int pack_split(mf_matrix m, Layout &L, int cls, int listed)
 {
     hipStream_t st = stream();
     const size_t rows = (size_t)m->tilem * m->B;
     uint8_t *codes = nullptr;
     int *d_n = nullptr;
-    MF_HIP(hipMallocAsync((void **)&codes, (size_t)m->tilenum + 1, st));
-    MF_HIP(hipMallocAsync((void **)&d_n, sizeof(int), st));
-    MF_HIP(hipMalloc((void **)&L.exc, sizeof(PlaneExc) * (size_t)listed));
-    MF_HIP(hipMemsetAsync(d_n, 0, sizeof(int), st));
-    int rc = classes_device(m, L.tau, L.allow_mask, codes);
-    if (rc) return rc;
-    const unsigned nb = (unsigned)((m->tilem + 255) / 256);
+    int n = 0;
+    std::vector<PlaneExc> e(listed);
+    auto pack = [&]() -> int {
+        if (hipMallocAsync((void **)&codes, (size_t)m->tilenum + 1, st) != hipSuccess ||
+            hipMallocAsync((void **)&d_n, sizeof(int), st) != hipSuccess ||
+            hipMalloc((void **)&L.exc, sizeof(PlaneExc) * (size_t)listed) != hipSuccess) {
+            (void)hipGetLastError();  // a failed allocation leaves its pointer null
+            return MF_E_NOMEM;
+        }
+        MF_HIP(hipMemsetAsync(d_n, 0, sizeof(int), st));
+        int rc = classes_device(m, L.tau, L.allow_mask, codes);
+        if (rc) return rc;
+        const unsigned nb = (unsigned)((m->tilem + 255) / 256);
 #define MF_SPLIT(BB)                                                                                                    \
     k_planes_split<BB><<<nb, 256, 0, st>>>(m->d_tile_ptr, m->tilem, m->d_tile_start, m->d_tile_columnidx, m->d_rowtmp,  \
                                            m->d_Blockcsr_Val, m->d_Tile_csr_Col, codes, m->d_st, cls, rows, L.planes,   \
                                            L.exc, listed, d_n)
-    if (m->B == 16) MF_SPLIT(16);
-    else if (m->B == 8) MF_SPLIT(8);
-    else MF_SPLIT(32);
+        if (m->B == 16) MF_SPLIT(16);
+        else if (m->B == 8) MF_SPLIT(8);
+        else MF_SPLIT(32);
 #undef MF_SPLIT
-    MF_HIP(hipGetLastError());
-    int n = 0;
-    std::vector<PlaneExc> e(listed);
-    MF_HIP(hipMemcpyAsync(&n, d_n, sizeof(int), hipMemcpyDeviceToHost, st));
-    MF_HIP(hipMemcpyAsync(e.data(), L.exc, sizeof(PlaneExc) * e.size(), hipMemcpyDeviceToHost, st));
-    MF_HIP(hipStreamSynchronize(st));
-    MF_HIP(hipFreeAsync(codes, st));
-    MF_HIP(hipFreeAsync(d_n, st));
-    if (n != listed) return fail(MF_E_FORMAT, "stencil planes: classes changed");
+        MF_HIP(hipGetLastError());
+        MF_HIP(hipMemcpyAsync(&n, d_n, sizeof(int), hipMemcpyDeviceToHost, st));
+        MF_HIP(hipMemcpyAsync(e.data(), L.exc, sizeof(PlaneExc) * e.size(), hipMemcpyDeviceToHost, st));
+        MF_HIP(hipStreamSynchronize(st));
+        return n == listed ? MF_OK : fail(MF_E_FORMAT, "stencil planes: classes changed");
+    };
+    int rc = pack();
+    if (codes) (void)hipFreeAsync(codes, st);
+    if (d_n) (void)hipFreeAsync(d_n, st);
+    if (rc) return rc;
     std::sort(e.begin(), e.end(), [](const PlaneExc &a, const PlaneExc &b) {
         return a.row != b.row ? a.row < b.row : a.cls != b.cls ? a.cls < b.cls : a.off < b.off;
     });
@@ -1070,7 +1083,7 @@ int ensure_planes(mf_matrix m, Layout &L)
     const int cls = planes_class(L, &listed);
     if (cls < 0) return MF_OK;
     int rc = find_stencil(m);
-    if (rc || !m->st_L) return rc;
+    if (rc || m->st_L <= 0) return rc;
     const size_t rows = (size_t)m->tilem * m->B;
     const size_t bytes = rows * plane_row_bytes(cls, m->st_L);
     // planes hold a value for every row and offset: worth it where that is
@@ -1078,19 +1091,26 @@ int ensure_planes(mf_matrix m, Layout &L)
     // most rows use a few entries of
     if (bytes > L.blob_bytes + L.blob_bytes / 4) return MF_OK;
     hipStream_t st = stream();
-    if (hipMalloc((void **)&L.planes, bytes) != hipSuccess) {  // short of memory: the slabs serve
-        (void)hipGetLastError();
-        L.planes = nullptr;
-        return MF_OK;
-    }
-    MF_HIP(hipMemsetAsync(L.planes, 0, bytes, st));
-    if (!listed) {
+    auto fill = [&]() -> int {
+        if (hipMalloc((void **)&L.planes, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            L.planes = nullptr;
+            return MF_E_NOMEM;
+        }
+        MF_HIP(hipMemsetAsync(L.planes, 0, bytes, st));
+        if (listed) return pack_split(m, L, cls, listed);
         k_planes_pack<<<(unsigned)((m->rowA + 255) / 256), 256, 0, st>>>(m->d_rowptr, m->d_col, m->d_val, m->rowA, m->d_st,
                                                                          cls, rows, L.planes);
         MF_HIP(hipGetLastError());
-    } else {
-        rc = pack_split(m, L, cls, listed);
-        if (rc) return rc;
+        return MF_OK;
+    };
+    rc = fill();
+    if (rc) {
+        if (L.planes) (void)hipFree(L.planes);
+        if (L.exc) (void)hipFree(L.exc);
+        L.planes = nullptr;
+        L.exc = nullptr;
+        return rc == MF_E_NOMEM ? MF_OK : rc;  // short of memory: the slabs serve
     }
     L.planes_cls = cls;
     return MF_OK;
