@@ -197,7 +197,8 @@ int mf_matrix_get_info(mf_matrix m, mf_matrix_info *info);
  * whose rows share their column offsets (stencils) stores one table of
  * offsets instead of an index per entry (pattern slab), and where all rows
  * of the matrix draw from one short table of offsets and the layout holds one
- * class, the solvers run on planes of values without indices.  1, 2 or 4 = that
+ * class (or one and few entries of narrower ones: BiCGSTAB alone), the solvers run on
+ * planes of values without indices where those are the faster.  1, 2 or 4 = that
  * form where it fits, else the next wider one, and no pattern slabs or planes.
  * Layouts already built are released.  Results are bit-identical across
  * forms.  No reference counterpart (the reference stores four-byte columns

@@ -503,7 +503,9 @@ template <int B, int IW, int CM = CM_ALL> struct Slabs {
 };
 
 // CG (Hestenes-Stiefel with s = A p carried by recurrence): registers hold
-// x and p of the thread's rows, LDS holds r and s.  Per iteration: [r
+// x and p of the thread's rows, LDS holds s, and r on slabs; on stencil planes
+// registers hold r too, and x stays in the caller's buffer beyond X_REGS_ROWS
+// rows per thread.  Per iteration: [r
 // published, (r, r) reduced] -> convergence test -> w = A r, s = w + beta s,
 // p = r + beta p and (p, s) in the same pass -> reduce (p, s) -> x, r updates
 // -> publish r, reduce (r, r).  The denominator (p, A p) is summed directly
@@ -1427,9 +1429,10 @@ template <int B> KernelChoice pick_tile_acc64(int iw, int method, long long rows
                      : pick_kernel_acc64<B, 4>(method, rows_per_wg, G);
 }
 
-// Resident kernels on the stencil planes of class cls (a64: low-precision
-// values summed in FP64, see pick_kernel_acc64).  Rows per thread go up to 28
-// for CG: x, p and r of a row in registers, s in LDS.
+// Resident kernels on the stencil planes of one class.  Rows per thread go up to
+// 36 for CG: p and r of a row in registers, s in LDS, x in registers up to 16
+// rows and in the caller's buffer beyond.  BiCGSTAB holds five vectors in
+// registers and stops at 8.
 template <class M> KernelChoice pick_stencil_kernel(int method, long long rows_per_wg)
 {
     KernelChoice k;
@@ -1452,6 +1455,7 @@ template <class M> KernelChoice pick_stencil_kernel(int method, long long rows_p
     }
     return k;
 }
+// Small systems, low-precision values summed in FP64 (see pick_kernel_acc64).
 template <class M> KernelChoice pick_stencil_acc64(int method, long long rows_per_wg, int G)
 {
     KernelChoice k;

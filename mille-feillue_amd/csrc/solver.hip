@@ -599,8 +599,10 @@ static int launch_inner(mf_matrix m, const Layout &L, const Layout *L64, int met
     if (!kc.fn) kc = pick(m->B, L.iw, method, (long long)trw * m->B, false, layout_cm(L), G);
     if (!kc.fn) return fail(MF_E_UNSUPPORTED, "no persistent kernel for this tile size and index form");
     // streaming the vectors of a system whose rows fit on chip is switched
-    // off: two runs that forced it on small grids ended with a GPU fault
-    // whose cause is not known
+    // off: two runs that forced it on small grids ended with a GPU fault.  One
+    // cause was found since and mended (padding gathers of tile rows past the
+    // last one, up to 16 KB beyond the vector); whether it was theirs is not
+    // known
     if (o.vectors == MF_VECTORS_HBM && !kc.streamed)
         return fail(MF_E_UNSUPPORTED, "vectors in HBM only for systems beyond register/LDS residency");
     if (o.vectors == MF_VECTORS_ONCHIP && kc.streamed)

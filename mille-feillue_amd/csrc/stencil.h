@@ -9,7 +9,7 @@
 // of one row after the other, so a wave reads contiguous blocks and nothing is
 // read but values: row r's entry at table position j sits at position j,
 // positions it lacks hold value 0.  Loads of one row do not depend on each
-// other, and the loop keeps `depth` rows in flight.  Entries keep their order
+// other, and the loop keeps two rows, or four quads, in flight.  Entries keep their order
 // and zeros add nothing to a sum that starts at +0, so the sums are bit
 // for bit those of the slabs.
 //
