@@ -151,8 +151,9 @@ static int layout_cm(const Layout &L)
 // pick_stencil_kernel), no listed entries in CG, and, in solves of one workgroup, not planes of quads
 // (tables other than 5 or 7 offsets) where the slabs are in LDS with up to two rows
 // per thread, nor with more rows in FP64 on more than 8 offsets or BiCGSTAB on
-// FP16.  There every product waits for LDS alone, and the slabs' loop has two
-// rows' quads in flight; measured, planes / slabs, ms: 27-point BiCGSTAB of 512 rows
+// FP16.  There a product waits for LDS alone, and the planes' loop waits in every
+// quad for a scalar load of its four offsets besides, on the counter that its
+// LDS reads share; measured, planes / slabs, ms: 27-point BiCGSTAB of 512 rows
 // FP64 0.238 / 0.195, 729 rows FP16 0.531 / 0.407, 1728 rows FP64 0.687 / 0.602;
 // 3 offsets, 1000 rows, CG 0.199 / 0.166; on the other side, slabs too long for
 // LDS: 13 offsets, 1000 rows, FP64 BiCGSTAB 0.87 of the slabs' time, 9 offsets, 2000
